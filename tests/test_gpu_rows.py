@@ -1,0 +1,108 @@
+"""MatMulNBits of up to 64 rows in any float types (k_gemv_rows) on the GPU, at the sizes where its
+launch shapes, remainders and operand paths change, against float64 sums over the oracle's weights.
+
+Bound per output, S = sum |a w| of its products: 2^-20 S for the f32 sums (K up to a few thousand in
+chunks of 32, each partial sum rounding by 2^-24 of its value) and the weights' own f32 rounding,
+plus half a unit in the last place of the dot's and of Y's type (2^-11 f16, 2^-8 bf16)."""
+
+import zlib
+
+import numpy as np
+import pytest
+
+from oracle import oracle as o
+from synth import nbits_weight
+from test_gpu_nbits import as_f64, host_float
+from transmuter_amd import PackedWeight
+from transmuter_amd.device import bf16_host
+from transmuter_amd.quantized import matmul_nbits
+
+pytestmark = pytest.mark.gpu
+
+HALF_ULP = {"f32": 2.0 ** -24, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}
+
+
+def typed(x, dtype):
+    h = host_float(x, dtype)
+    return bf16_host(h) if dtype == "bf16" else h
+
+
+def check(ctx, a, a_dtype, w_dtype, k, n, bits, block, zp, bias_dtype=None, seed=0):
+    rng = np.random.default_rng(seed)
+    b, s32, z = nbits_weight(rng, k, n, bits, block, zp=zp, scale_dtype=np.float32)
+    scales = typed(s32, w_dtype)
+    w = PackedWeight.upload(ctx, b, scales, z, k=k, n=n, bits=bits, block_size=block, weight_dtype=w_dtype)
+    bias = None if bias_dtype is None else typed(rng.standard_normal(n), bias_dtype)
+    y_t = matmul_nbits(ctx.put(a), w, bias)
+    y = as_f64(y_t.numpy(), y_t.dtype)
+    dense = o.dequantize_weight(b, as_f64(scales, w_dtype).astype(np.float32), z, k, n, bits, block, w_dtype)
+    dense = np.asarray(dense, np.float64)
+    af = as_f64(a, a_dtype)
+    with np.errstate(invalid="ignore"):
+        ref = af @ dense.T
+    dot_dtype = a_dtype if a_dtype == w_dtype else "f32"
+    bound = 2.0 ** -20 * (np.abs(af) @ np.abs(dense).T) + HALF_ULP[dot_dtype] * np.abs(ref)
+    if bias is not None:
+        ref = ref + as_f64(bias, bias_dtype)
+    bound = bound + HALF_ULP[y_t.dtype] * np.abs(ref) + (2.0 ** -24 if "f16" in (dot_dtype, y_t.dtype) else 0)
+    w.free()
+    return y, ref, bound
+
+
+def chunk(bits):
+    return 512 // bits
+
+
+# Launch shapes: tiles x 16-row sets against 256, 512, 1024 and 2048 workgroups; up to 8 chunks and more.
+SHAPES = [(1, 16, 1), (16, 17, 8), (17, 40, 9), (33, 300, 17), (64, 1024, 33), (1, 4097, 3), (16, 4160, 11), (8, 33000, 2),
+          (31, 2064, 9), (48, 2704, 2), (32, 5000, 3), (20, 9000, 2), (30, 16500, 2), (64, 16400, 2), (20, 66000, 1)]
+TYPES = [("f16", "f16"), ("bf16", "bf16"), ("f32", "f32")]
+
+
+@pytest.mark.parametrize("a_dtype,w_dtype", TYPES)
+@pytest.mark.parametrize("m,n,chunks", SHAPES)
+def test_launch_shapes(ctx, m, n, chunks, a_dtype, w_dtype):
+    k = chunks * chunk(4) - 24  # a partial last chunk and block
+    print(f"rows m={m} n={n} k={k} {a_dtype}", flush=True)
+    rng = np.random.default_rng(m * 1000 + n)
+    a = typed(rng.standard_normal((m, k)), a_dtype)
+    # (An f32 bias keeps up to 16 rows of f16 from the f16 decode GEMV.)
+    bias = "f32" if a_dtype == "f16" and m <= 16 else None
+    y, ref, bound = check(ctx, a, a_dtype, w_dtype, k, n, 4, 32, "packed", bias, seed=n)
+    assert (np.abs(y - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("bits,block", [(2, 16), (2, 64), (4, 16), (4, 64), (4, 256), (8, 16), (8, 32), (8, 128)])
+@pytest.mark.parametrize("zp", ["none", "packed", "float"])
+@pytest.mark.parametrize("a_dtype,w_dtype", TYPES + [("f32", "f16"), ("f16", "f32"), ("bf16", "f32"), ("f16", "bf16")])
+def test_operand_paths(ctx, bits, block, zp, a_dtype, w_dtype):
+    case = (bits, block, zp, a_dtype, w_dtype)
+    rng = np.random.default_rng(zlib.crc32(repr(case).encode()))
+    m, n = int(rng.choice([3, 16, 21, 70])), int(rng.choice([19, 150]))
+    k = chunk(bits) * int(rng.integers(1, 12)) + 8 * int(rng.integers(0, 4))
+    bias = [None, "f32", w_dtype][int(rng.integers(3))]
+    print(f"operand path {case} m={m} n={n} k={k} bias={bias}", flush=True)
+    a = typed(rng.standard_normal((m, k)), a_dtype)
+    y, ref, bound = check(ctx, a, a_dtype, w_dtype, k, n, bits, block, zp, bias, seed=m)
+    if m > 64 and a_dtype != w_dtype or (m > 64 and zp == "float") or (m > 64 and a_dtype == "f32"):
+        bound = bound + 2.0 ** -14 * np.abs(ref).max()  # the prefill GEMM keeps 16 bits of each f32 factor
+    assert (np.abs(y - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("a_dtype,w_dtype", [("f32", "f32"), ("f32", "f16"), ("bf16", "bf16"), ("f16", "f16")])
+def test_wide_range_infinities_and_nan(ctx, a_dtype, w_dtype):
+    """Values over the type's whole range, and rows with an infinity or a NaN: those rows' outputs are
+    the float64 sum's (infinite or NaN), and no other row sees them."""
+    rng = np.random.default_rng(5)
+    m, k, n = 20, 520, 64
+    top = 4 if a_dtype == "f16" else 30
+    a = rng.standard_normal((m, k)) * 10.0 ** rng.uniform(-top, top, (m, 1))
+    a[3, 17], a[4, 40], a[5, 300] = np.inf, -np.inf, np.nan
+    a = typed(a, a_dtype)
+    y, ref, bound = check(ctx, a, a_dtype, w_dtype, k, n, 4, 32, "none", seed=9)
+    special = [3, 4, 5]
+    assert not np.isfinite(y[special]).any()
+    rest = [i for i in range(m) if i not in special]
+    limit = {"f16": 65504.0}.get(a_dtype if a_dtype == w_dtype else "f32", 3.4e38)
+    fits = np.abs(ref[rest]) < limit
+    assert (np.abs(y[rest] - ref[rest])[fits] <= bound[rest][fits]).all()

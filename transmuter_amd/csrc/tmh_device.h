@@ -191,6 +191,104 @@ __device__ __forceinline__ half8_t unpack_step(const uint4_t& w, int i, half2_t 
   return out;
 }
 
+// x and y with the odd rows of lanes (16-31, 48-63) of x and the even rows of y exchanged.
+__device__ __forceinline__ void swap_rows(uint32_t& x, uint32_t& y) {
+  const auto p = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+  x = p[0];
+  y = p[1];
+}
+// x and y with the upper half (lanes 32-63) of x and the lower half of y exchanged.
+__device__ __forceinline__ void swap_halves(uint32_t& x, uint32_t& y) {
+  const auto p = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+  x = p[0];
+  y = p[1];
+}
+
+// A lane's 16 weight bytes of a chunk (k-group g of its row) turned into the words of the natural
+// steps: step i's words of lane row g are those of k = 32 i + 8 g.
+template <int BITS>
+__device__ __forceinline__ uint4_t natural_words(const uint4_t& w) {
+  uint32_t a = w[0], b = w[1], c = w[2], d = w[3];
+  if constexpr (BITS == 4) {  // word i of group G is step G's word of lane row i
+    swap_halves(a, c);
+    swap_halves(b, d);
+    swap_rows(a, b);
+    swap_rows(c, d);
+  } else {  // 8 bits: words 2j, 2j+1 of group G are step G/2's words of lane row 2 (G % 2) + j
+    swap_rows(a, c);
+    swap_rows(b, d);
+    swap_halves(a, c);
+    swap_halves(b, d);
+  }
+  return uint4_t{a, b, c, d};
+}
+
+// A value held per k-group handed to the lanes of the natural steps: out[i] is the value of the
+// k-group that step i's eight weights of this lane come from.
+template <int BITS>
+__device__ __forceinline__ void natural_params(uint32_t x, uint32_t* out) {
+  uint32_t a = x, b = x;
+  swap_rows(a, b);  // a: groups 0 0 2 2, b: groups 1 1 3 3
+  if constexpr (BITS == 4) {
+    out[0] = a;
+    out[2] = a;
+    swap_halves(out[0], out[2]);
+    out[1] = b;
+    out[3] = b;
+    swap_halves(out[1], out[3]);
+  } else {
+    swap_halves(a, b);  // a: groups 0 0 1 1, b: groups 2 2 3 3
+    out[0] = a;
+    out[1] = b;
+  }
+}
+
+// scale * (q - zero) of the eight values q of step i, in k order: one fma each over the f16 numbers
+// 1024 + q that the packed values become under the exponent of 0x6400 (as in unpack_step; the
+// nibbles at bits 4-7 give 1024 + 16 q, whose scale is scale / 16). Each product and sum is exact
+// (for a bf16 scale below 2^117, or scale 1), so the fma's one rounding rounds nothing.
+template <int BITS>
+__device__ __forceinline__ void natural_values(const uint4_t& w, int i, float scale, float zero, float (&q)[8]) {
+  // (Held from constant folding: a scale of 1 known to the compiler becomes a conversion and a
+  // subtraction, two instructions for the one v_fma_mix_f32.)
+  asm volatile("" : "+v"(scale));
+  const float c = -(1024.f + zero) * scale;
+  uint32_t pr[4];
+  if constexpr (BITS == 4) {
+    const uint32_t x = w[i];
+    const uint32_t magic = __builtin_amdgcn_readfirstlane(0x64006400u);
+    pr[0] = and_or(x, 0x000F000Fu, magic);
+    pr[1] = and_or(x, 0x00F000F0u, magic);
+    pr[2] = and_or(x >> 8, 0x000F000Fu, magic);
+    pr[3] = and_or(x >> 8, 0x00F000F0u, magic);
+  } else if constexpr (BITS == 8) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      pr[2 * h] = __builtin_amdgcn_perm(0x64646464u, w[2 * i + h], 0x04010400u);
+      pr[2 * h + 1] = __builtin_amdgcn_perm(0x64646464u, w[2 * i + h], 0x04030402u);
+    }
+  } else {
+    const uint32_t x = w[i >> 1] >> (8 * (i & 1));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) pr[j] = ((x >> (2 * j)) & 0x00030003u) | 0x64006400u;
+  }
+  const float scale16 = scale * 0.0625f, c16 = -(64.f + zero) * scale;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const half2_t h = __builtin_bit_cast(half2_t, pr[j]);
+    const bool high = BITS == 4 && (j & 1);
+    q[2 * j] = fmaf(static_cast<float>(h[0]), high ? scale16 : scale, high ? c16 : c);
+    q[2 * j + 1] = fmaf(static_cast<float>(h[1]), high ? scale16 : scale, high ? c16 : c);
+  }
+}
+
+// Two f32 values rounded to bf16 (to nearest even) in one word, the first in the low half.
+__device__ __forceinline__ uint32_t pack_bf16_rne(float a, float b) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  const bf16x2_t p = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
+  return __builtin_bit_cast(uint32_t, p);
+}
+
 // XOR swizzle of the 16-byte pieces of LDS rows that 16 lanes read as MFMA fragments (lane r of a
 // lane group reads row r, all lanes the same piece): piece p of row r sits in slot
 // p ^ frag_swizzle<PPR>(r). The values were found by timing ds_read_b128 over candidate tables on

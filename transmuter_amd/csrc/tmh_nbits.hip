@@ -10,11 +10,13 @@
 // Kernels
 //   k_dequant         the {N, K} weights, bit-exact, in any float type
 //   k_gemv_dec        (tmh_gemv.h) decode GEMV for M <= 16, f16 Y (an f16 bias or none)
-//   k_gemv_f16        f16 A and f16 weights, M <= 16*MT per block row: every lane unpacks its
+//   k_gemv_rows       (tmh_rows.h) up to 64 rows of A in any float types
+//   k_gemv_f16        (A rows off 16-byte boundaries, or weights past 32-bit offsets)
+//                     f16 A and f16 weights, M <= 16*MT per block row: every lane unpacks its
 //                     16 bytes in registers into exact f16 weights (q - zero) * scale and feeds
 //                     v_mfma_f32_16x16x32_f16; four wavefronts split K and add through LDS
 //   k_gemm_f16        the same fragments for larger M, 128x128 tiles per workgroup
-//   k_matmul_general  any float types and float zero points, f32 FMA on the vector ALUs
+//   k_matmul_general  the same exceptions in the other float types, f32 FMA on the vector ALUs
 #include <algorithm>
 #include <cstdio>
 #include <mutex>
@@ -1242,15 +1244,8 @@ void launch_gemv_u(const tmh_weight* w, const MatArgs& a, hipStream_t s, int wav
 // Chunks per wavefront round (U) and wavefronts per block: up to 16 wavefronts, each with
 // 1, 2 or 4 chunk loads in flight, so that K of up to 64 chunks needs one round.
 template <int BITS, int MT, bool HAS_ZP, bool SPLIT>
-void launch_gemv(const tmh_weight* w, const MatArgs& a, hipStream_t s, int num_cus) {
+void launch_gemv(const tmh_weight* w, const MatArgs& a, hipStream_t s) {
   const int64_t c = w->nchunks;
-  // The decode GEMV (tmh_gemv.hip): f16 Y without bias or with an f16 one, aligned A, 32-bit
-  // offsets.
-  if (MT == 1 && a.y_dt == TMH_F16 && a.dot_dt == TMH_F16 && (!a.bias || a.bias_dt == TMH_F16) &&
-      decode_gemv_ok(w, a.M, a.lda, a.ldy, a.a, a.y)) {
-    launch_decode_gemv(w, a.a, a.M, a.lda, a.y, a.ldy, s, num_cus, a.bias);
-    return;
-  }
   if (c <= 16) {
     launch_gemv_u<BITS, MT, HAS_ZP, SPLIT, 1>(w, a, s, static_cast<int>(c));
   } else if (c <= 32) {
@@ -1445,14 +1440,24 @@ bool fast_path(const tmh_weight* w, const MatArgs& a) {
   return a.a_dt == TMH_F16 && w->wdtype == TMH_F16 && w->zp_kind != TMH_ZP_FLOAT;
 }
 
-// The operand path of the LDS-tiled prefill GEMM for a call, or -1 where it does not apply: M > 64
-// and 32-bit buffer offsets over the weights; f16 A with f16 weights (GM_F16) and bf16 A with bf16
+// Rows of A that the LDS-tiled GEMM takes: over 64, and from 33 on (17 for vocabulary-sized N) where
+// 16-bit operands meet so many columns that its 64-row tiles fill half the CUs without a split of K
+// (those calls need no scratch memory). f16 q4 in graph replays, this GEMM against k_gemv_rows:
+// 2048->22016, M = 64 19.0 / 24.9 us (M = 24: 18 / 14.8), 1024->18000, M = 64 11.1 / 13-15,
+// 1024->151936, M = 32 35.1 / 48.7; below, 4096->12288 (768 tiles), M = 64 32.8 / 27-30.
+bool gemm_rows(const tmh_weight* w, const MatArgs& a) {
+  return a.M > 64 || (a.M > (w->ntiles >= 4096 ? 16 : 32) && w->ntiles >= 1024 && a.a_dt == w->wdtype &&
+                      a.a_dt != TMH_F32 && a.a_vec && w->zp_kind != TMH_ZP_FLOAT);
+}
+
+// The operand path of the LDS-tiled prefill GEMM for a call, or -1 where it does not apply: enough
+// rows (gemm_rows) and 32-bit buffer offsets over the weights; f16 A with f16 weights (GM_F16) and bf16 A with bf16
 // weights (GM_BF16, one parameter entry per lane) without float zero points read A as given and
 // need it aligned, with 32-bit offsets over it (and a tile of rows past M); every other float
 // combination goes through GM_SPLIT (one parameter entry per lane, 32-bit offsets over its hi and
 // lo rows) unless the call cannot give it scratch memory for them (no_split_a).
 int gemm_mode(const tmh_weight* w, const MatArgs& a) {
-  if (a.M <= 64 || w->ntiles * w->nchunks * 1024 + 16 * w->nchunks * 1024 >= (int64_t(1) << 31)) return -1;
+  if (!gemm_rows(w, a) || w->ntiles * w->nchunks * 1024 + 16 * w->nchunks * 1024 >= (int64_t(1) << 31)) return -1;
   const bool direct_f16 = a.a_dt == TMH_F16 && w->wdtype == TMH_F16 && w->zp_kind != TMH_ZP_FLOAT;
   const bool direct_bf16 = a.a_dt == TMH_BF16 && w->wdtype == TMH_BF16 && w->zp_kind != TMH_ZP_FLOAT;
   if (direct_f16 || direct_bf16) {
@@ -1465,6 +1470,9 @@ int gemm_mode(const tmh_weight* w, const MatArgs& a) {
   if ((a.M + kGemmBM) * kp * 2 >= (int64_t(1) << 31)) return -1;
   return GM_SPLIT;
 }
+
+// Most bytes of partial sums a call's plan may keep: none up to 64 rows (see gemm_rows).
+size_t split_cap_of(const MatArgs& a) { return a.M > 64 ? a.split_cap : 0; }
 
 // Scratch memory of one call: GM_SPLIT's hi and lo rows of A, then the f32 partial sums of a plan
 // that splits K (splits * M * N), each 256-byte aligned; zeros where the call needs none.
@@ -1483,38 +1491,38 @@ GemmScratch gemm_scratch(const tmh_ctx* ctx, const tmh_weight* w, const MatArgs&
   const int mode = gemm_mode(w, a);
   if (mode < 0) return g;
   if (mode == GM_SPLIT) g.a_split = split_a_bytes(w, a.M);
-  const GemmPlan p = plan_gemm(a.M, w->N, w->ntiles, w->nchunks, w->bits, cus_of(ctx), a.split_cap, mode);
+  const GemmPlan p = plan_gemm(a.M, w->N, w->ntiles, w->nchunks, w->bits, cus_of(ctx), split_cap_of(a), mode);
   if (p.splits > 1) g.partials = static_cast<size_t>(p.splits) * static_cast<size_t>(a.M) * static_cast<size_t>(w->N) * sizeof(float);
   return g;
 }
 
 template <int BITS, bool HAS_ZP, bool SPLIT>
-void launch_fast_variant(tmh_ctx* ctx, const tmh_weight* w, const MatArgs& a, hipStream_t s) {
+void launch_fast_variant(const tmh_weight* w, const MatArgs& a, hipStream_t s) {
   if (a.M <= 16) {
-    launch_gemv<BITS, 1, HAS_ZP, SPLIT>(w, a, s, ctx->num_cus);
+    launch_gemv<BITS, 1, HAS_ZP, SPLIT>(w, a, s);
   } else if (a.M <= 32) {
-    launch_gemv<BITS, 2, HAS_ZP, SPLIT>(w, a, s, ctx->num_cus);
+    launch_gemv<BITS, 2, HAS_ZP, SPLIT>(w, a, s);
   } else if (a.M <= 64 || BITS == 2) {
-    launch_gemv<BITS, 4, HAS_ZP, SPLIT>(w, a, s, ctx->num_cus);
+    launch_gemv<BITS, 4, HAS_ZP, SPLIT>(w, a, s);
   } else if constexpr (BITS != 2) {
     launch_gemm<BITS, HAS_ZP, SPLIT>(w, a, s);
   }
 }
 
 template <int BITS>
-void launch_fast_bits(tmh_ctx* ctx, const tmh_weight* w, const MatArgs& a, hipStream_t s) {
+void launch_fast_bits(const tmh_weight* w, const MatArgs& a, hipStream_t s) {
   const bool zp = w->zp_kind == TMH_ZP_PACKED;
   const bool split = split_params(w);
-  if (zp && split) launch_fast_variant<BITS, true, true>(ctx, w, a, s);
-  else if (zp) launch_fast_variant<BITS, true, false>(ctx, w, a, s);
-  else if (split) launch_fast_variant<BITS, false, true>(ctx, w, a, s);
-  else launch_fast_variant<BITS, false, false>(ctx, w, a, s);
+  if (zp && split) launch_fast_variant<BITS, true, true>(w, a, s);
+  else if (zp) launch_fast_variant<BITS, true, false>(w, a, s);
+  else if (split) launch_fast_variant<BITS, false, true>(w, a, s);
+  else launch_fast_variant<BITS, false, false>(w, a, s);
 }
 
 // The prefill GEMM on operand path `mode` (gemm_mode), with GM_SPLIT's hi/lo rows of A made first.
 template <int BITS>
 void launch_gemm_bits(tmh_ctx* ctx, const tmh_weight* w, const MatArgs& a, hipStream_t s, int mode) {
-  const GemmPlan p = plan_gemm(a.M, w->N, w->ntiles, w->nchunks, BITS, cus_of(ctx), a.split_cap, mode);
+  const GemmPlan p = plan_gemm(a.M, w->N, w->ntiles, w->nchunks, BITS, cus_of(ctx), split_cap_of(a), mode);
   const bool zp = w->zp_kind == TMH_ZP_PACKED;
   if (mode == GM_F16) {
     const GemmA ga{a.a, w->K, a.lda};
@@ -2116,17 +2124,33 @@ int launch_matmul(tmh_ctx* ctx, const tmh_weight* w, const MatArgs& a, hipStream
     }
     return check_launch(ctx, "k_gemm_lds");
   }
-  if (fast_path(w, a)) {
-    switch (w->bits) {
-      case 2: launch_fast_bits<2>(ctx, w, a, s); break;
-      case 4: launch_fast_bits<4>(ctx, w, a, s); break;
-      default: launch_fast_bits<8>(ctx, w, a, s);
-    }
-    return check_launch(ctx, "k_gemv_f16/k_gemm_f16");
+  // The f16 and f32 decode GEMVs where they apply, then k_gemv_rows.
+  if (fast_path(w, a) && a.y_dt == TMH_F16 && a.dot_dt == TMH_F16 && (!a.bias || a.bias_dt == TMH_F16) &&
+      decode_gemv_ok(w, a.M, a.lda, a.ldy, a.a, a.y)) {
+    launch_decode_gemv(w, a.a, a.M, a.lda, a.y, a.ldy, s, ctx->num_cus, a.bias);
+    return check_launch(ctx, "k_gemv_dec/k_gemv_dot");
   }
   if (a.a_dt == TMH_F32 && a.y_dt == TMH_F32 && !a.bias && decode_gemv_f32_ok(w, a.M, a.lda, a.ldy, a.a)) {
     launch_decode_gemv_f32(w, a.a, a.M, a.lda, a.y, a.ldy, s);
     return check_launch(ctx, "k_gemv_f32");
+  }
+  if ((a.M <= 64 || !fast_path(w, a)) && gemv_rows_ok(w, a.a, a.a_dt, std::min<int64_t>(a.M, 64), a.lda)) {
+    // (More than 64 rows come here where the GEMM has no build for the parameters, bf16 or f32 with
+    // several blocks in a lane's group, or no 32-bit offsets over A: in launches of 64 rows.)
+    for (int64_t m = 0; m < a.M; m += 64)
+      launch_gemv_rows(w, static_cast<const uint8_t*>(a.a) + m * a.lda * dtype_size(a.a_dt), a.a_dt,
+                       std::min<int64_t>(a.M - m, 64), a.lda, a.bias, a.bias_dt,
+                       static_cast<uint8_t*>(a.y) + m * a.ldy * dtype_size(a.y_dt), a.y_dt, a.dot_dt, a.ldy, s,
+                       ctx->num_cus);
+    return check_launch(ctx, "k_gemv_rows");
+  }
+  if (fast_path(w, a)) {
+    switch (w->bits) {
+      case 2: launch_fast_bits<2>(w, a, s); break;
+      case 4: launch_fast_bits<4>(w, a, s); break;
+      default: launch_fast_bits<8>(w, a, s);
+    }
+    return check_launch(ctx, "k_gemv_f16/k_gemm_f16");
   }
   switch (w->bits) {
     case 2: launch_general_bits<2>(w, a, s); break;
