@@ -111,3 +111,19 @@ def _check(ctx, case):
     ref = o.dequantize_linear(x, scale, zero, axis=axis, block_size=bs)
     assert got.shape == ref.shape and got.dtype == ref.dtype
     assert np.array_equal(got.reshape(-1).view(np.uint8), np.ascontiguousarray(ref).reshape(-1).view(np.uint8))
+
+
+# 2- and 4-byte x, per tensor or along a last axis of a multiple of 4 (four elements per thread), and
+# beside it the sizes that k_dequantize_linear4 keeps: an odd axis, an odd total, one parameter group.
+WIDE = [((3, 1028), 1, "axis"), ((5, 4), 1, "axis"), ((2, 3, 64), 2, "axis"), ((1024,), 0, "tensor"), ((257, 4), 0, "tensor"),
+        ((7, 1027), 1, "axis"), ((9, 13), 0, "tensor"), ((6, 8), 0, "axis")]
+
+
+@pytest.mark.parametrize("xdt,sdt", [("s32", "f32"), ("s32", "f16"), ("s32", "bf16"), ("u16", "f32"), ("s16", "bf16"),
+                                     ("f32", "f32"), ("f16", "f16")])
+@pytest.mark.parametrize("with_zero", [False, True])
+@pytest.mark.parametrize("shape,axis,layout", WIDE)
+def test_wide_values(ctx, shape, axis, layout, xdt, sdt, with_zero):
+    case = (shape, axis, 0, layout, xdt, sdt, with_zero)
+    print(f"wide dequantize_linear {case}", flush=True)
+    _check(ctx, case)

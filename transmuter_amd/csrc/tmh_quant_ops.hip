@@ -456,6 +456,10 @@ __global__ __launch_bounds__(256) void k_dequantize_linear4(
   const uint32_t rem = e0 - o * per_outer;
   uint32_t d = rem / inner;
   uint32_t in = rem - d * inner;
+  // The four x values of a 4-byte type in one load where they are all there and aligned.
+  uint4_t raw = {0u, 0u, 0u, 0u};
+  const bool raw_x = (x_dt == TMH_S32 || x_dt == TMH_F32) && e0 + 4 <= total && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  if (raw_x) raw = *reinterpret_cast<const uint4_t*>(static_cast<const uint32_t*>(x) + e0);
   float out[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -466,11 +470,12 @@ __global__ __launch_bounds__(256) void k_dequantize_linear4(
       else if (mode == TMH_QPARAM_BLOCKED) p = (o * nb + d / bs) * inner + in;
       float v;
       if (x_int) {
-        uint32_t shifted = static_cast<uint32_t>(load_int_rt(x, x_dt, e));
+        uint32_t shifted = raw_x ? raw[j] : static_cast<uint32_t>(load_int_rt(x, x_dt, e));
         if (zero) shifted -= static_cast<uint32_t>(load_int_rt(zero, zero_dt, p));
         v = static_cast<float>(static_cast<int32_t>(shifted));
       } else {
-        v = load_float_rt(x, x_dt, e);
+        const uint32_t bits = raw[j];
+        v = raw_x ? __builtin_bit_cast(float, bits) : load_float_rt(x, x_dt, e);
         if (zero) v = v - load_float_rt(zero, zero_dt, p);
       }
       out[j] = v * load_float_rt(scale, scale_dt, p);
@@ -556,6 +561,104 @@ __global__ __launch_bounds__(256) void k_dequantize_linear_b4(const uint32_t* __
     __builtin_nontemporal_store(u32x2_t{h[0] | (static_cast<uint32_t>(h[1]) << 16), h[2] | (static_cast<uint32_t>(h[3]) << 16)},
                                 reinterpret_cast<u32x2_t*>(y) + t);
   }
+}
+
+// DequantizeLinear of 2- and 4-byte values (integers or floats; XS: their bytes) with per-tensor
+// parameters or parameters along the last axis (AXIS, dim % 4 == 0), zero points of x's type or none:
+// four elements per thread from one 8- or 16-byte load, their scales and zero points from one load
+// each, one 8- or 16-byte store; the arithmetic of k_dequantize_linear4. Bound by memory: the s32
+// sums of a 2048 x 2048 MatMulInteger to f32, 33.6 MB, take 6.9 us (4.9 TB/s); k_dequantize_linear4,
+// whose four 4-byte loads a thread each stride 16 bytes across the wavefront, took 12.9.
+template <int OUT, int XS, bool AXIS>
+__global__ __launch_bounds__(256) void k_dequantize_linear_w4(const void* __restrict__ x, int x_dt,
+                                                              const void* __restrict__ scale,
+                                                              const void* __restrict__ zero, uint32_t dim,
+                                                              void* __restrict__ y, uint32_t quads) {
+  const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+  if (t >= quads) return;
+  auto raw4 = [](const void* p, uint32_t quad, uint32_t (&r)[4]) {
+    if constexpr (XS == 4) {
+      const uint4_t v = static_cast<const uint4_t*>(p)[quad];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r[j] = v[j];
+    } else {
+      const uint2 v = static_cast<const uint2*>(p)[quad];
+      r[0] = v.x & 0xFFFFu;
+      r[1] = v.x >> 16;
+      r[2] = v.y & 0xFFFFu;
+      r[3] = v.y >> 16;
+    }
+  };
+  uint32_t xr[4], zr[4];
+  raw4(x, t, xr);
+  float sc[4];
+  if constexpr (AXIS) {
+    const uint32_t d4 = (t * 4u) % dim / 4u;  // the four elements share a row: parameters d .. d+3
+    if constexpr (OUT == DT_F32) {
+      const float4_t v = static_cast<const float4_t*>(scale)[d4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sc[j] = v[j];
+    } else {
+      const uint2 v = static_cast<const uint2*>(scale)[d4];
+      const uint32_t w[2] = {v.x, v.y};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const auto h = static_cast<uint16_t>(w[j / 2] >> (16 * (j % 2)));
+        sc[j] = OUT == DT_F16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
+      }
+    }
+    if (zero) raw4(zero, d4, zr);
+  } else {
+    const float s0 = load_as_f32<OUT>(scale, 0);
+    const uint32_t z0 = !zero ? 0u : XS == 4 ? *static_cast<const uint32_t*>(zero) : *static_cast<const uint16_t*>(zero);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      sc[j] = s0;
+      zr[j] = z0;
+    }
+  }
+  // A raw value as the type's s32 value, or (float types) as f32.
+  auto int_of = [&](uint32_t r) -> uint32_t {
+    return x_dt == TMH_S16 ? static_cast<uint32_t>(static_cast<int32_t>(static_cast<int16_t>(r))) : r;
+  };
+  auto float_of = [&](uint32_t r) -> float {
+    if constexpr (XS == 4) return __builtin_bit_cast(float, r);
+    return x_dt == TMH_F16 ? f16_bits_to_f32(static_cast<uint16_t>(r)) : bf16_bits_to_f32(static_cast<uint16_t>(r));
+  };
+  float out[4];
+  if (x_dt == TMH_F32 || x_dt == TMH_F16 || x_dt == TMH_BF16) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[j] = (zero ? float_of(xr[j]) - float_of(zr[j]) : float_of(xr[j])) * sc[j];
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint32_t shifted = int_of(xr[j]);  // s32 subtraction, wrapping
+      if (zero) shifted -= int_of(zr[j]);
+      out[j] = static_cast<float>(static_cast<int32_t>(shifted)) * sc[j];
+    }
+  }
+  if constexpr (OUT == DT_F32) {
+    __builtin_nontemporal_store(float4_t{out[0], out[1], out[2], out[3]}, static_cast<float4_t*>(y) + t);
+  } else {
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    uint16_t h[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h[j] = OUT == DT_F16 ? f32_to_f16_bits(out[j]) : f32_to_bf16_bits(out[j]);
+    __builtin_nontemporal_store(u32x2_t{h[0] | (static_cast<uint32_t>(h[1]) << 16), h[2] | (static_cast<uint32_t>(h[3]) << 16)},
+                                static_cast<u32x2_t*>(y) + t);
+  }
+}
+
+template <int OUT>
+void launch_dql_w4(const void* x, int x_dt, int x_size, const void* scale, const void* zero, bool axis, uint32_t dim,
+                   void* y, uint32_t quads, hipStream_t s) {
+  const dim3 grid((quads + 255) / 256);
+  if (x_size == 4)
+    axis ? k_dequantize_linear_w4<OUT, 4, true><<<grid, 256, 0, s>>>(x, x_dt, scale, zero, dim, y, quads)
+         : k_dequantize_linear_w4<OUT, 4, false><<<grid, 256, 0, s>>>(x, x_dt, scale, zero, dim, y, quads);
+  else
+    axis ? k_dequantize_linear_w4<OUT, 2, true><<<grid, 256, 0, s>>>(x, x_dt, scale, zero, dim, y, quads)
+         : k_dequantize_linear_w4<OUT, 2, false><<<grid, 256, 0, s>>>(x, x_dt, scale, zero, dim, y, quads);
 }
 
 template <int OUT, bool SIGNED>
@@ -1076,6 +1179,19 @@ int tmh_dequantize_linear(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t ou
               : launch_dql_b4<DT_F32, false>(d_x, d_scale, d_zero, axis, d32, d_y, quads, s);
       }
       return check_launch(ctx, "k_dequantize_linear_b4");
+    }
+    // 2- and 4-byte x with the same parameter layouts, its zero points of the same type.
+    const int x_size = dtype_size(x_dtype);
+    if ((x_size == 2 || x_size == 4) && (!d_zero || zero_dtype == x_dtype) && (mode == TMH_QPARAM_TENSOR || axis) &&
+        total % 4 == 0 && total / 4 < (int64_t{1} << 30) && aligned(d_x, 4 * x_size) && aligned(d_y, 4 * out_bytes) &&
+        (!axis || aligned(d_scale, 4 * out_bytes)) && (!axis || !d_zero || aligned(d_zero, 4 * x_size))) {
+      const auto quads = static_cast<uint32_t>(total / 4), d32 = static_cast<uint32_t>(dim);
+      switch (scale_dtype) {
+        case TMH_F16: launch_dql_w4<DT_F16>(d_x, x_dtype, x_size, d_scale, d_zero, axis, d32, d_y, quads, s); break;
+        case TMH_BF16: launch_dql_w4<DT_BF16>(d_x, x_dtype, x_size, d_scale, d_zero, axis, d32, d_y, quads, s); break;
+        default: launch_dql_w4<DT_F32>(d_x, x_dtype, x_size, d_scale, d_zero, axis, d32, d_y, quads, s);
+      }
+      return check_launch(ctx, "k_dequantize_linear_w4");
     }
   }
   if (total < (int64_t{1} << 31) - 4) {
