@@ -386,15 +386,25 @@ constexpr int kGemmBM = 256;  // largest tile height: bounds the A rows a launch
 //           f32's exponent range), the weights are dequantized in f32 and rounded to their own type
 //           WT as the reference does, then split the same way, and each product takes three bf16
 //           MFMAs (hi*hi + lo*hi + hi*lo; the dropped lo*lo term is below 2^-16 of each product).
-enum : int { GM_F16 = 0, GM_BF16 = 1, GM_SPLIT = 2 };
+//  GM_INT   f32 A and f32 weights of 4 or 8 bits in blocks of 32 and more (an f32 export as it comes),
+//           packed or no zero points: q - zero is a whole number of at most 8 bits and so exact in
+//           bf16; the weight words trade lanes (natural_words) so that a step's 32 values of k lie in
+//           one block, and the block's f32 scale multiplies the step's f32 sums: two MFMAs per product
+//           (the hi and lo rows of A) and four FMAs a lane, in place of three MFMAs and the splitting
+//           of every weight, and no rounding of the weights. 509 x 1024 -> 6144 (kernel alone, traced):
+//           32.3 -> 27.3 us; the four projections of a layer of that width, with the splitting of A and
+//           the split-K sums, 121.6 -> 97.5 us; relative error against float64 4.5e-6 -> 2.5e-6.
+enum : int { GM_F16 = 0, GM_BF16 = 1, GM_SPLIT = 2, GM_INT = 3 };
+// The paths that take A as hi and lo rows of bf16.
+constexpr bool splits_a(int mode) { return mode == GM_SPLIT || mode == GM_INT; }
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
-// LDS of one workgroup: the double-buffered A tile (two tiles, hi and lo, for GM_SPLIT), or
+// LDS of one workgroup: the double-buffered A tile (two tiles, hi and lo, where A is split), or
 // (KS = 2) the partial sums of half the wavefronts after the k-loop, whichever is larger.
 template <int BITS, int BM, int KS = 1, int MODE = GM_F16>
 constexpr size_t gemm_lds_bytes() {
-  constexpr size_t a_tiles = 2 * static_cast<size_t>(BM) * (512 / BITS) * 2 * (MODE == GM_SPLIT ? 2 : 1);
+  constexpr size_t a_tiles = 2 * static_cast<size_t>(BM) * (512 / BITS) * 2 * (splits_a(MODE) ? 2 : 1);
   constexpr size_t partial = KS > 1 ? static_cast<size_t>(BM) * 128 * sizeof(float) : 0;
   return a_tiles > partial ? a_tiles : partial;
 }
@@ -550,8 +560,8 @@ __device__ __forceinline__ void gemm_lds(
   constexpr int MTW = TALL ? BM / 16 : 8;
   constexpr int NTW = TALL ? 2 : 4;
   static_assert(MODE == GM_F16 || (TALL && !SPLIT), "the bf16 paths use the tall layout, one parameter per lane");
-  constexpr int ABUF = BM * ROWB * (MODE == GM_SPLIT ? 2 : 1);  // LDS bytes of one A buffer (hi, then lo)
-  constexpr int SES = MODE == GM_SPLIT && WT == DT_F32 ? 4 : 2;  // bytes per stored scale
+  constexpr int ABUF = BM * ROWB * (splits_a(MODE) ? 2 : 1);  // LDS bytes of one A buffer (hi, then lo)
+  constexpr int SES = splits_a(MODE) && WT == DT_F32 ? 4 : 2;  // bytes per stored scale
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -575,12 +585,12 @@ __device__ __forceinline__ void gemm_lds(
   const uint32_t kb1 = kb0 + chunks_per_split < nch ? kb0 + chunks_per_split : nch;
 
   const auto a_rsrc = buffer_rsrc(A, static_cast<uint32_t>(M * lda * 2));
-  const auto alo_rsrc = buffer_rsrc(static_cast<const uint8_t*>(A) + (MODE == GM_SPLIT ? M * lda * 2 : 0),
-                                    MODE == GM_SPLIT ? static_cast<uint32_t>(M * lda * 2) : 0u);
+  const auto alo_rsrc = buffer_rsrc(static_cast<const uint8_t*>(A) + (splits_a(MODE) ? M * lda * 2 : 0),
+                                    splits_a(MODE) ? static_cast<uint32_t>(M * lda * 2) : 0u);
   const auto q_rsrc = buffer_rsrc(qt, static_cast<uint32_t>(ntiles * nchunks * 1024));
   const uint32_t n_params = static_cast<uint32_t>(ntiles * nchunks * nbc * 16);
   const auto s_rsrc = buffer_rsrc(sc, n_params * SES);
-  const uint32_t z_bytes = MODE == GM_SPLIT ? (zk == TMH_ZP_FLOAT ? n_params * 4 : zk == TMH_ZP_PACKED ? zp_byte<BITS>(n_params) : 0u)
+  const uint32_t z_bytes = splits_a(MODE) ? (zk == TMH_ZP_FLOAT ? n_params * 4 : zk == TMH_ZP_PACKED ? zp_byte<BITS>(n_params) : 0u)
                                             : (HAS_ZP ? zp_byte<BITS>(n_params) : 0u);
   const auto z_rsrc = buffer_rsrc(zp, z_bytes);
   const uint32_t zsh = zp_shift<BITS>(r);  // every entry this lane reads is one of row r
@@ -602,10 +612,10 @@ __device__ __forceinline__ void gemm_lds(
       for (int s2 = 0; s2 < LOADS; ++s2)
         if (s2 >= s_lo && s2 < s_hi) {
           lds_dma16(a_rsrc, base + s2 * RPI * ROWB, a_off(s2), kb * (CW * 2));
-          if constexpr (MODE == GM_SPLIT) lds_dma16(alo_rsrc, base + BM * ROWB + s2 * RPI * ROWB, a_off(s2), kb * (CW * 2));
+          if constexpr (splits_a(MODE)) lds_dma16(alo_rsrc, base + BM * ROWB + s2 * RPI * ROWB, a_off(s2), kb * (CW * 2));
         }
     } else {
-      // (GM_SPLIT's A is zero-padded to whole chunks by k_split_a, so it never comes here.)
+      // (Split A is zero-padded to whole chunks by k_split_a, so it never comes here.)
       // A k-block that reaches past K: through registers, zero past K. The whole offset is in
       // the VGPR operand so the buffer range check covers it.
 #pragma unroll
@@ -627,6 +637,7 @@ __device__ __forceinline__ void gemm_lds(
     uint4_t w[NTW];
     uint32_t s[NJ][NTW];
     uint32_t z[NJ][NTW];
+    float4_t sq[MODE == GM_INT ? LSTEPS : 1][NTW];  // GM_INT: scales of the lane's four columns in its steps
   };
   auto load_b = [&](uint32_t kb, BStage& st, int t_lo = 0, int t_hi = 1 << 30) {
     const uint32_t kofs = kb * static_cast<uint32_t>(nbc) * 16;
@@ -638,6 +649,15 @@ __device__ __forceinline__ void gemm_lds(
       for (int j = 0; j < NJ; ++j) {
         uint32_t e = p_base + nt * p_tstep;
         if constexpr (SPLIT) e += static_cast<uint32_t>(((g * GW + 8 * j) >> bsc_shift) - ((g * GW) >> bsc_shift)) * 16;
+        if constexpr (MODE == GM_INT) {
+#pragma unroll
+          for (int li = 0; li < LSTEPS; ++li)
+            st.sq[li][nt] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                s_rsrc, ((static_cast<uint32_t>(t0 + nt) * nch * nbc + ((32 * (kh * LSTEPS + li)) >> bsc_shift)) * 16 + 4 * g) * 4,
+                kofs * 4, 0));
+          st.z[j][nt] = __builtin_amdgcn_raw_buffer_load_b8(z_rsrc, zp_byte<BITS>(e), zp_byte<BITS>(kofs), 0);
+          continue;
+        }
         if constexpr (SES == 4) st.s[j][nt] = __builtin_amdgcn_raw_buffer_load_b32(s_rsrc, e * 4, kofs * 4, 0);
         else st.s[j][nt] = __builtin_amdgcn_raw_buffer_load_b16(s_rsrc, e * 2, kofs * 2, 0);
         if constexpr (MODE == GM_SPLIT) {
@@ -695,7 +715,75 @@ __device__ __forceinline__ void gemm_lds(
   };
   auto compute = [&](int buf, const BStage& st, bool more, uint32_t kbn, BStage& nst) {
     const uint8_t* abase = lds + buf * ABUF + (wm * 128 + r) * ROWB;
-    if constexpr (MODE != GM_F16) {
+    if constexpr (MODE == GM_INT) {
+      uint4_t wn[NTW];
+      uint32_t zn[NTW][STEPS];
+#pragma unroll
+      for (int nt = 0; nt < NTW; ++nt) {
+        wn[nt] = natural_words<BITS>(st.w[nt]);
+        natural_params<BITS>(zk == TMH_ZP_PACKED ? zp_field<BITS>(st.z[0][nt], zsh) : 1u << (BITS - 1), zn[nt]);
+      }
+      auto steps = [&](auto khc) {
+        constexpr int KH = decltype(khc)::value;
+#pragma unroll
+        for (int li = 0; li < LSTEPS; ++li) {
+          const int i = KH * LSTEPS + li;
+          if (more) issue(li, kbn, buf ^ 1, nst);
+          uint4_t b[NTW];
+          float4_t prev[NTW];
+#pragma unroll
+          for (int nt = 0; nt < NTW; ++nt) {
+            float q[8];
+            natural_values<BITS>(wn[nt], i, 1.f, static_cast<float>(zn[nt][i]), q);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[nt][j] = pack_bf16_rne(q[2 * j], q[2 * j + 1]);
+          }
+          const int slot = a_slot<BITS>(r, 4 * i + g) * 16;
+          uint4_t ah = *reinterpret_cast<const uint4_t*>(abase + slot);
+          uint4_t al = *reinterpret_cast<const uint4_t*>(abase + BM * ROWB + slot);
+#pragma unroll
+          for (int mt = 0; mt < MTW; ++mt) {
+            uint4_t ahn{}, aln{};
+            if (mt + 1 < MTW) {
+              ahn = *reinterpret_cast<const uint4_t*>(abase + (mt + 1) * 16 * ROWB + slot);
+              aln = *reinterpret_cast<const uint4_t*>(abase + BM * ROWB + (mt + 1) * 16 * ROWB + slot);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            float4_t sum[NTW];
+#pragma unroll
+            for (int nt = 0; nt < NTW; ++nt) sum[nt] = gm_mma<MODE>(b[nt], al, float4_t{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int nt = 0; nt < NTW; ++nt) sum[nt] = gm_mma<MODE>(b[nt], ah, sum[nt]);
+            // The sums of fragment mt are scaled behind the MFMAs of fragment mt + 1.
+            if (mt > 0) {
+#pragma unroll
+              for (int nt = 0; nt < NTW; ++nt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[mt - 1][nt][e] = fmaf(st.sq[li][nt][e], prev[nt][e], acc[mt - 1][nt][e]);
+            }
+#pragma unroll
+            for (int nt = 0; nt < NTW; ++nt) prev[nt] = sum[nt];
+            __builtin_amdgcn_sched_barrier(0);
+            if (mt + 1 < MTW) {
+              ah = ahn;
+              al = aln;
+            }
+          }
+#pragma unroll
+          for (int nt = 0; nt < NTW; ++nt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[MTW - 1][nt][e] = fmaf(st.sq[li][nt][e], prev[nt][e], acc[MTW - 1][nt][e]);
+        }
+      };
+      if constexpr (KS == 1) {
+        steps(std::integral_constant<int, 0>{});
+      } else if (kh == 0) {
+        steps(std::integral_constant<int, 0>{});
+      } else {
+        steps(std::integral_constant<int, 1>{});
+      }
+      return;
+    } else if constexpr (MODE != GM_F16) {
       // The bf16 paths (tall layout): the step pipeline of the f16 path, with the weights
       // dequantized through f32 and, for GM_SPLIT, the hi and lo parts of A and of the weights
       // (three MFMAs per product).
@@ -973,7 +1061,7 @@ __device__ __forceinline__ void gemm_lds(
         *reinterpret_cast<uint2*>(static_cast<uint16_t*>(Y) + m * ldy + n) = pack4(v);
         continue;
       }
-      if (MODE == GM_SPLIT && y_dt == DT_F32 && dot_dt == DT_F32 && !bias && vec_out && n + 4 <= N &&
+      if (splits_a(MODE) && y_dt == DT_F32 && dot_dt == DT_F32 && !bias && vec_out && n + 4 <= N &&
           (reinterpret_cast<uintptr_t>(Y) & 15) == 0) {
         *reinterpret_cast<float4_t*>(static_cast<float*>(Y) + m * ldy + n) = v;
         continue;
@@ -1025,8 +1113,10 @@ __global__ __launch_bounds__(256) void k_split_a(const void* __restrict__ A, int
     const float x0 = k < K ? load_as_f32<ADT>(A, m * lda + k) : 0.f;
     const float x1 = k + 1 < K ? load_as_f32<ADT>(A, m * lda + k + 1) : 0.f;
     const uint32_t h = pack_bf16(x0, x1);
+    const float h0 = __builtin_bit_cast(float, h << 16), h1 = __builtin_bit_cast(float, h & 0xFFFF0000u);
     hi[j] = h;
-    lo[j] = pack_bf16(x0 - __builtin_bit_cast(float, h << 16), x1 - __builtin_bit_cast(float, h & 0xFFFF0000u));
+    // (An infinite hi part is the whole value: inf - inf would make it a NaN.)
+    lo[j] = pack_bf16(fabsf(h0) == INFINITY ? 0.f : x0 - h0, fabsf(h1) == INFINITY ? 0.f : x1 - h1);
   }
   *reinterpret_cast<uint4_t*>(out + m * Kp + k0) = hi;
   *reinterpret_cast<uint4_t*>(out + (M + m) * Kp + k0) = lo;
@@ -1294,7 +1384,7 @@ int cus_of(const tmh_ctx* ctx) { return ctx->num_cus > 0 ? ctx->num_cus : 256; }
 
 // gemm_lds_bytes at run time.
 size_t gemm_lds_bytes_rt(int bits, int bm, int ks, int mode) {
-  const size_t a_tiles = 2 * static_cast<size_t>(bm) * (512 / bits) * 2 * (mode == GM_SPLIT ? 2 : 1);
+  const size_t a_tiles = 2 * static_cast<size_t>(bm) * (512 / bits) * 2 * (splits_a(mode) ? 2 : 1);
   const size_t partial = ks > 1 ? static_cast<size_t>(bm) * 128 * sizeof(float) : 0;
   return std::max(a_tiles, partial);
 }
@@ -1306,13 +1396,13 @@ bool shape_built(int bits, int bm, int wn, int ks, int mode) {
   if (gemm_lds_bytes_rt(bits, bm, ks, mode) > 128 * 1024) return false;
   const bool eight = (bm == 128 || bm == 64) && ((wn == 2 && ks == 2) || (wn == 4 && ks == 1));
   if (mode == GM_BF16) return eight;
-  if (mode == GM_SPLIT) return eight && wn == 2;
+  if (splits_a(mode)) return eight && wn == 2;
   return true;
 }
 
 // split_cap bounds the f32 partial sums a split plan keeps (splits * M * N * 4 bytes): plans
 // beyond it are not considered, a forced one included. The bf16 path is priced at the f16 rates
-// and GM_SPLIT at a third of them (three MFMAs per product).
+// and GM_SPLIT and GM_INT at a third and half of them (three and two MFMAs per product).
 GemmPlan plan_gemm(int64_t M, int64_t N, int64_t ntiles, int64_t nchunks, int bits, int cus,
                    size_t split_cap = SIZE_MAX, int mode = GM_F16) {
   auto fits = [&](int64_t splits) {
@@ -1320,7 +1410,7 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t ntiles, int64_t nchunks, int bi
            static_cast<double>(splits) * static_cast<double>(M) * static_cast<double>(N) * 4.0 <= static_cast<double>(split_cap);
   };
   const double cw = 512.0 / bits;
-  const double slow = mode == GM_SPLIT ? 3.0 : 1.0;
+  const double slow = mode == GM_SPLIT ? 3.0 : mode == GM_INT ? 2.0 : 1.0;
   GemmPlan best{128, 2, 1, static_cast<int>(nchunks), 2};
   double best_t = 1e30;
   for (const GemmShape& sh : kGemmShapes) {
@@ -1468,6 +1558,8 @@ int gemm_mode(const tmh_weight* w, const MatArgs& a) {
   if (split_params(w) || a.no_split_a) return -1;
   const int64_t kp = w->nchunks * chunk_weights(w->bits);
   if ((a.M + kGemmBM) * kp * 2 >= (int64_t(1) << 31)) return -1;
+  if (a.a_dt == TMH_F32 && w->wdtype == TMH_F32 && w->zp_kind != TMH_ZP_FLOAT && w->bits != 2 && w->block_size >= 32)
+    return GM_INT;
   return GM_SPLIT;
 }
 
@@ -1490,7 +1582,7 @@ GemmScratch gemm_scratch(const tmh_ctx* ctx, const tmh_weight* w, const MatArgs&
   GemmScratch g;
   const int mode = gemm_mode(w, a);
   if (mode < 0) return g;
-  if (mode == GM_SPLIT) g.a_split = split_a_bytes(w, a.M);
+  if (splits_a(mode)) g.a_split = split_a_bytes(w, a.M);
   const GemmPlan p = plan_gemm(a.M, w->N, w->ntiles, w->nchunks, w->bits, cus_of(ctx), split_cap_of(a), mode);
   if (p.splits > 1) g.partials = static_cast<size_t>(p.splits) * static_cast<size_t>(a.M) * static_cast<size_t>(w->N) * sizeof(float);
   return g;
@@ -1549,6 +1641,10 @@ void launch_gemm_bits(tmh_ctx* ctx, const tmh_weight* w, const MatArgs& a, hipSt
     default: k_split_a<DT_F32><<<sgrid, 256, 0, s>>>(a.a, a.M, w->K, a.lda, kp, split_rows);
   }
   const GemmA ga{split_rows, kp, kp};
+  if (mode == GM_INT) {
+    if constexpr (BITS != 2) launch_gemm_plan<BITS, false, false, GM_INT, DT_F32>(w, a, ga, s, p);
+    return;
+  }
   switch (w->wdtype) {
     case TMH_F16: launch_gemm_plan<BITS, false, false, GM_SPLIT, DT_F16>(w, a, ga, s, p); break;
     case TMH_BF16: launch_gemm_plan<BITS, false, false, GM_SPLIT, DT_BF16>(w, a, ga, s, p); break;
@@ -2221,8 +2317,8 @@ int tmh_matmul_nbits_noalloc(tmh_ctx* ctx, const tmh_weight* w, const void* d_a,
   // The call keeps its scratch memory within the scratch area: GM_SPLIT's rows of A when they fit
   // (else the general kernel runs), then the partial sums of the best plan that fits in the rest
   // (where tmh_matmul_nbits's plan would need more: fewer splits of K, or none).
-  if (gemm_mode(w, a) == GM_SPLIT && split_a_bytes(w, a.M) > kNoallocScratchBytes) a.no_split_a = true;
-  const size_t rows_a = gemm_mode(w, a) == GM_SPLIT ? split_a_bytes(w, a.M) : 0;
+  if (splits_a(gemm_mode(w, a)) && split_a_bytes(w, a.M) > kNoallocScratchBytes) a.no_split_a = true;
+  const size_t rows_a = splits_a(gemm_mode(w, a)) ? split_a_bytes(w, a.M) : 0;
   a.split_cap = kNoallocScratchBytes - rows_a;
   const GemmScratch g = gemm_scratch(ctx, w, a);
   if (const size_t need = g.total()) {
