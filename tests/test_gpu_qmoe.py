@@ -105,13 +105,14 @@ def test_random_qmoe(ctx, seed):
     _check_qmoe(ctx, case)
 
 
-def _check_qmoe(ctx, case):
+def _check_qmoe(ctx, case, skew=0.0):
     dtype, e, k, t, h, n1, act, fusion, fc3, bits, bs, zp, bias, limit = case
     rng = np.random.default_rng(zlib.crc32(repr(case).encode()))
     npdt = np.float16 if dtype == "f16" else np.float32
     inter = n1 if (act != "swiglu" or fc3) else n1 // 2
     x = rng.standard_normal((t, h)).astype(npdt)
     router = rng.standard_normal((t, e)).astype(np.float32)
+    router[:, 0] += skew  # draws the tokens to expert 0
     w1, s1, z1 = _weights(rng, e, n1, h, bits, bs, zp, dtype)
     w2, s2, z2 = _weights(rng, e, h, inter, bits, bs, zp, dtype)
     w3, s3, z3 = _weights(rng, e, n1, h, bits, bs, zp, dtype) if fc3 else (None, None, None)
@@ -254,3 +255,27 @@ def test_qmoe_rejects_expert_rows_off_the_16_row_tiles(ctx, n1, h):
     assert status == ERR_UNSUPPORTED and "multiples of 16" in message, message
     fc1.free()
     fc2.free()
+
+
+# Few rows an expert and few experts (at most 32 reached; 64 from 16 chunks of K on): the product over
+# items of 16 rows. Epilogues, odd tile counts (the last workgroup's second tile is none), one chunk of
+# K and partial ones, K split unevenly, parameters that change within a lane's group, and the sizes
+# beside the rule (33 experts, over eight rows an expert); up to 32 tokens routed and planned by one
+# workgroup, 33 by two launches.
+FEW_CASES = [
+    ("f16", 1, 1, 8, 64, 48, "silu", 0, False, 4, 32, False, False, 0.0),
+    ("f16", 4, 2, 16, 144, 80, "swiglu", 0, True, 4, 32, True, False, 0.0),
+    ("f16", 4, 2, 17, 144, 80, "swiglu", 0, True, 4, 32, True, False, 0.0),
+    ("f16", 32, 4, 32, 528, 96, "gelu", 0, False, 8, 64, True, True, 0.0),
+    ("f16", 32, 4, 33, 1040, 208, "swiglu", 2, False, 4, 16, True, True, 7.0),
+    ("f16", 33, 1, 40, 272, 64, "relu", 0, False, 4, 128, False, False, 0.0),
+    ("f16", 64, 8, 8, 2064, 64, "swiglu", 0, True, 4, 64, False, False, 0.0),
+    ("f16", 16, 3, 40, 400, 1200, "identity", 0, False, 8, 16, False, True, 0.0),
+]
+
+
+@pytest.mark.parametrize("case", FEW_CASES, ids=lambda c: "{}_E{}_k{}_T{}_H{}_N{}_{}_b{}_bs{}".format(*c[:7], c[9], c[10]))
+@pytest.mark.parametrize("skew", [0.0, 6.0])
+def test_qmoe_few_rows(ctx, case, skew):
+    print(f"qmoe few rows {case} skew={skew}", flush=True)
+    _check_qmoe(ctx, case, skew)

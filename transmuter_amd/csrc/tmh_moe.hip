@@ -32,6 +32,8 @@ using namespace tmh;
 namespace {
 
 constexpr int kMoeRows = 32;  // rows per work item of the general product
+// Tokens up to which one workgroup routes and plans (k_moe_route_plan): two for each of its wavefronts.
+constexpr int kFusedRouteTokens = 32;
 
 // ------------------------------------------------------------------ routing and grouping
 
@@ -70,11 +72,9 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 // empty, then its lowest lane), and sets that key to 0; lane r keeps the round's value and index.
 // (The body; k_moe_route and its stamping build k_moe_route_tl below are the kernels.)
 template <int RDT, int EJ>
-__device__ __forceinline__ void moe_route(const void* __restrict__ router, int T, int E, int k,
+__device__ __forceinline__ void moe_route(const void* __restrict__ router, int t, int E, int k,
                                           int* __restrict__ topi, float* __restrict__ topw) {
   const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (t >= T) return;
   uint32_t key[EJ];
 #pragma unroll
   for (int j = 0; j < EJ; ++j) {
@@ -130,17 +130,15 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
   return v;
 }
 
-// One workgroup of 1024 threads (thread e for expert e): rows per expert, expert offsets (exclusive
-// prefix of the counts), the list of work items (expert << 16 | item of the expert, `rows` rows
-// each; the items with the most 16-row m-tiles first), and the position of every (token, slot)
-// row in expert order (perm) with its inverse
-// (slot_pos). Each thread loads four rows' experts per round before its LDS atomics; up to 4096
+// One workgroup of 1024 threads (thread e for expert e): rows per expert, their exclusive prefix
+// sums, the list of work items (expert, first sorted row, up to `rows` rows; the items with the most
+// 16-row m-tiles first), and the position of every (token, slot) row in expert order (perm) with its
+// inverse (slot_pos). Each thread loads four rows' experts per round before its LDS atomics; up to 4096
 // rows the ids stay in registers from the count to the placement. The prefix sums run per
 // wavefront in DPP steps, then across the 16 wavefronts.
 // (The body; k_moe_plan and k_moe_plan_tl below are the kernels.)
-__device__ __forceinline__ void moe_plan(int* __restrict__ counts, int E, int rows, const int* __restrict__ topi,
-                                         int Tk, int* __restrict__ offsets, int* __restrict__ items,
-                                         int* __restrict__ n_items, int* __restrict__ perm,
+__device__ __forceinline__ void moe_plan(int E, int rows, const int* __restrict__ topi, int Tk,
+                                         int4* __restrict__ items, int* __restrict__ n_items, int* __restrict__ perm,
                                          int* __restrict__ slot_pos) {
   constexpr int R = 4;
   __shared__ int first_s[1024], fill[1024], wsum_r[16], wsum_i[16], cls_next[5];
@@ -162,7 +160,6 @@ __device__ __forceinline__ void moe_plan(int* __restrict__ counts, int E, int ro
   __syncthreads();
   const int c = fill[e];
   const int nb = (c + rows - 1) / rows;
-  if (e < E) counts[e] = c;
   // Work items in descending order of their 16-row m-tiles (the heaviest first: the products'
   // workgroups run in item order, so the last ones to start are light). An expert's items are
   // full but its last (q_last m-tiles); the order within a class is the atomics' (any order
@@ -183,7 +180,6 @@ __device__ __forceinline__ void moe_plan(int* __restrict__ counts, int E, int ro
     si += wsum_i[w2];
   }
   const int first_row = sr - c;
-  if (e < E) offsets[e] = first_row;
   if (e == 1023) *n_items = si;
   if (e == 0) {  // each class's first item position, the classes in descending order
     int run = 0;
@@ -197,8 +193,8 @@ __device__ __forceinline__ void moe_plan(int* __restrict__ counts, int E, int ro
   fill[e] = 0;
   __syncthreads();
   if (e < E && nb > 0) {
-    for (int b = 0; b + 1 < nb; ++b) items[atomicAdd(&cls_next[q_full], 1)] = (e << 16) | b;
-    items[atomicAdd(&cls_next[q_last], 1)] = (e << 16) | (nb - 1);
+    for (int b = 0; b + 1 < nb; ++b) items[atomicAdd(&cls_next[q_full], 1)] = make_int4(e, first_row + b * rows, rows, 0);
+    items[atomicAdd(&cls_next[q_last], 1)] = make_int4(e, first_row + (nb - 1) * rows, c - (nb - 1) * rows, 0);
   }
   const bool held = Tk <= 1024 * R;
   for (int base = 0; base < Tk; base += 1024 * R) {
@@ -224,7 +220,8 @@ __device__ __forceinline__ void moe_plan(int* __restrict__ counts, int E, int ro
 template <int RDT, int EJ>
 __global__ __launch_bounds__(256) void k_moe_route(const void* __restrict__ router, int T, int E, int k,
                                                    int* __restrict__ topi, float* __restrict__ topw) {
-  moe_route<RDT, EJ>(router, T, E, k, topi, topw);
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t < T) moe_route<RDT, EJ>(router, t, E, k, topi, topw);
 }
 
 template <int RDT, int EJ>
@@ -232,25 +229,37 @@ __global__ __launch_bounds__(256) void k_moe_route_tl(const void* __restrict__ r
                                                       int* __restrict__ topi, float* __restrict__ topw,
                                                       uint32_t* __restrict__ tl) {
   const TlStart t0 = tl_clock();
-  moe_route<RDT, EJ>(router, T, E, k, topi, topw);
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t < T) moe_route<RDT, EJ>(router, t, E, k, topi, topw);
   tl_stamp(tl, t0);
 }
 
-__global__ __launch_bounds__(1024) void k_moe_plan(int* __restrict__ counts, int E, int rows, const int* __restrict__ topi,
-                                                   int Tk, int* __restrict__ offsets, int* __restrict__ items,
-                                                   int* __restrict__ n_items, int* __restrict__ perm,
-                                                   int* __restrict__ slot_pos) {
-  moe_plan(counts, E, rows, topi, Tk, offsets, items, n_items, perm, slot_pos);
+__global__ __launch_bounds__(1024) void k_moe_plan(int E, int rows, const int* __restrict__ topi, int Tk,
+                                                   int4* __restrict__ items, int* __restrict__ n_items,
+                                                   int* __restrict__ perm, int* __restrict__ slot_pos) {
+  moe_plan(E, rows, topi, Tk, items, n_items, perm, slot_pos);
 }
 
-__global__ __launch_bounds__(1024) void k_moe_plan_tl(int* __restrict__ counts, int E, int rows,
-                                                      const int* __restrict__ topi, int Tk, int* __restrict__ offsets,
-                                                      int* __restrict__ items, int* __restrict__ n_items,
+__global__ __launch_bounds__(1024) void k_moe_plan_tl(int E, int rows, const int* __restrict__ topi, int Tk,
+                                                      int4* __restrict__ items, int* __restrict__ n_items,
                                                       int* __restrict__ perm, int* __restrict__ slot_pos,
                                                       uint32_t* __restrict__ tl) {
   const TlStart t0 = tl_clock();
-  moe_plan(counts, E, rows, topi, Tk, offsets, items, n_items, perm, slot_pos);
+  moe_plan(E, rows, topi, Tk, items, n_items, perm, slot_pos);
   tl_stamp(tl, t0);
+}
+
+// Routing and planning of a few tokens in one workgroup of 16 wavefronts, a token each in turn: one
+// launch in place of two where each would be little but its launch (8 tokens, 128 experts: 4.7 + 3.9
+// us under the tracer).
+template <int RDT, int EJ>
+__global__ __launch_bounds__(1024) void k_moe_route_plan(const void* __restrict__ router, int T, int E, int k, int rows,
+                                                         int* __restrict__ topi, float* __restrict__ topw,
+                                                         int4* __restrict__ items, int* __restrict__ n_items,
+                                                         int* __restrict__ perm, int* __restrict__ slot_pos) {
+  for (int t = threadIdx.x >> 6; t < T; t += 16) moe_route<RDT, EJ>(router, t, E, k, topi, topw);
+  __syncthreads();  // the plan reads the choices back (this workgroup's own stores)
+  moe_plan(E, rows, topi, T * k, items, n_items, perm, slot_pos);
 }
 
 // ------------------------------------------------------------------ activations
@@ -298,11 +307,9 @@ struct MoeItem {
   int e, row0, rows;
 };
 
-__device__ __forceinline__ MoeItem moe_item(const int* items, int item, const int* offsets, const int* counts,
-                                            int rows) {
-  const int it = items[item];
-  const int e = it >> 16, b = it & 0xffff;
-  return MoeItem{e, offsets[e] + b * rows, min(rows, counts[e] - b * rows)};
+__device__ __forceinline__ MoeItem moe_item(const int4* items, int item) {
+  const int4 v = items[item];
+  return MoeItem{v.x, v.y, v.z};
 }
 
 // LDS slot of 16-byte piece `piece` of A row `row`: the XOR swizzle (frag_swizzle) under which
@@ -329,8 +336,7 @@ __device__ __forceinline__ void moe_gemm_f16(
     const uint4_t* __restrict__ qt2, const uint16_t* __restrict__ sc2, const uint8_t* __restrict__ zp2,
     int tile_off2, int ntiles, int nchunks, int nbc, int bsc_shift, int tiles_per_expert, int out_tiles, int gpw,
     const _Float16* __restrict__ A, int a_rows, int lda, const int* __restrict__ perm, int perm_div,
-    const int* __restrict__ items, const int* __restrict__ n_items, const int* __restrict__ offsets,
-    const int* __restrict__ counts, const void* __restrict__ bias1, const void* __restrict__ bias2, int bias_dt,
+    const int4* __restrict__ items, const int* __restrict__ n_items, const void* __restrict__ bias1, const void* __restrict__ bias2, int bias_dt,
     int bias_ld, int act, float alpha, float beta, float limit, _Float16* __restrict__ out, int ldo,
     const int* __restrict__ out_perm, uint32_t* __restrict__ tl) {
   const TlStart tl0 = TL ? tl_clock() : TlStart{0u, 0u};
@@ -349,7 +355,7 @@ __device__ __forceinline__ void moe_gemm_f16(
     if constexpr (TL) tl_stamp(tl, tl0);
     return;
   }
-  const MoeItem it = moe_item(items, blockIdx.y, offsets, counts, ROWS);
+  const MoeItem it = moe_item(items, blockIdx.y);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar branches, one LDS ring base
   const int r = lane & 15, g = lane >> 4;
@@ -522,14 +528,13 @@ __global__ __launch_bounds__(512) void k_moe_gemm_f16(
     const uint4_t* __restrict__ qt2, const uint16_t* __restrict__ sc2, const uint8_t* __restrict__ zp2,
     int tile_off2, int ntiles, int nchunks, int nbc, int bsc_shift, int tiles_per_expert, int out_tiles, int gpw,
     const _Float16* __restrict__ A, int a_rows, int lda, const int* __restrict__ perm, int perm_div,
-    const int* __restrict__ items, const int* __restrict__ n_items, const int* __restrict__ offsets,
-    const int* __restrict__ counts, const void* __restrict__ bias1, const void* __restrict__ bias2, int bias_dt,
+    const int4* __restrict__ items, const int* __restrict__ n_items, const void* __restrict__ bias1, const void* __restrict__ bias2, int bias_dt,
     int bias_ld, int act, float alpha, float beta, float limit, _Float16* __restrict__ out, int ldo,
     const int* __restrict__ out_perm) {
   moe_gemm_f16<BITS, HAS_ZP, SPLIT, EPI, MT, false>(
       qt, sc, zp, qt2, sc2, zp2, tile_off2, ntiles, nchunks, nbc, bsc_shift, tiles_per_expert, out_tiles, gpw, A, a_rows,
       lda, perm,
-      perm_div, items, n_items, offsets, counts, bias1, bias2, bias_dt, bias_ld, act, alpha, beta, limit, out, ldo, out_perm,
+      perm_div, items, n_items, bias1, bias2, bias_dt, bias_ld, act, alpha, beta, limit, out, ldo, out_perm,
       nullptr);
 }
 
@@ -539,15 +544,187 @@ __global__ __launch_bounds__(512) void k_moe_gemm_f16_tl(
     const uint4_t* __restrict__ qt2, const uint16_t* __restrict__ sc2, const uint8_t* __restrict__ zp2,
     int tile_off2, int ntiles, int nchunks, int nbc, int bsc_shift, int tiles_per_expert, int out_tiles, int gpw,
     const _Float16* __restrict__ A, int a_rows, int lda, const int* __restrict__ perm, int perm_div,
-    const int* __restrict__ items, const int* __restrict__ n_items, const int* __restrict__ offsets,
-    const int* __restrict__ counts, const void* __restrict__ bias1, const void* __restrict__ bias2, int bias_dt,
+    const int4* __restrict__ items, const int* __restrict__ n_items, const void* __restrict__ bias1, const void* __restrict__ bias2, int bias_dt,
     int bias_ld, int act, float alpha, float beta, float limit, _Float16* __restrict__ out, int ldo,
     const int* __restrict__ out_perm, uint32_t* __restrict__ tl) {
   moe_gemm_f16<BITS, HAS_ZP, SPLIT, EPI, MT, true>(
       qt, sc, zp, qt2, sc2, zp2, tile_off2, ntiles, nchunks, nbc, bsc_shift, tiles_per_expert, out_tiles, gpw, A, a_rows,
       lda, perm,
-      perm_div, items, n_items, offsets, counts, bias1, bias2, bias_dt, bias_ld, act, alpha, beta, limit, out, ldo, out_perm,
+      perm_div, items, n_items, bias1, bias2, bias_dt, bias_ld, act, alpha, beta, limit, out, ldo, out_perm,
       tl);
+}
+
+// The fast product for work items of up to 16 rows: the same sums and epilogue as moe_gemm_f16, for
+// calls that reach few experts, where reading their weights is nearly all there is to do and too few
+// workgroups read. A workgroup takes TN output tiles of one item and its NW wavefronts split K, each
+// with the weights and rows of its next chunk in flight while it computes one and no barrier until the
+// sums meet (moe_gemm_f16: a wavefront walks all of K of its tile, a barrier per chunk). A comes
+// straight from the L2 in the natural order of k (the lanes trade their weight words, natural_words),
+// so a lane's row may be any token's. Bound by the latency of item -> weights -> sums per workgroup,
+// then by the instructions that unpack (zero points known to be absent take a fifth of them away).
+// 2048/768 q4, graphless calls: one token, top 8 of 128 experts 41.4 -> 21.5 us, 8 tokens 58.6 -> 47.6
+// (fc1 and fc3 27.8 -> 23.9 us traced, fc2 17.2 -> 12.5).
+template <int BITS, bool HAS_ZP, bool SPLIT, int EPI, int TN, int NW>
+__global__ __launch_bounds__(64 * NW) void k_moe_rows(
+    const uint4_t* __restrict__ qt, const uint16_t* __restrict__ sc, const uint8_t* __restrict__ zp,
+    const uint4_t* __restrict__ qt2, const uint16_t* __restrict__ sc2, const uint8_t* __restrict__ zp2, int tile_off2,
+    int ntiles, int nchunks, int nbc, int bsc_shift, int tiles_per_expert, int out_tiles,
+    const _Float16* __restrict__ A, int a_rows, int lda, const int* __restrict__ perm, int perm_div,
+    const int4* __restrict__ items, const int* __restrict__ n_items, const void* __restrict__ bias1,
+    const void* __restrict__ bias2, int bias_dt, int bias_ld, int act, float alpha, float beta, float limit,
+    _Float16* __restrict__ out, int ldo, const int* __restrict__ out_perm) {
+  constexpr int CW = 512 / BITS;
+  constexpr int GW = CW / 4;
+  constexpr int STEPS = GW / 8;
+  constexpr int NJ = SPLIT ? STEPS : 1;
+  constexpr int NV = EPI == EPI_GLU ? 2 * TN : TN;  // weight tiles of a wavefront (EPI_GLU: first and second in turn)
+  static_assert(BITS != 2, "4- and 8-bit weights");
+  __shared__ float4_t red[NW * NV * 64];
+  if (static_cast<int>(blockIdx.y) >= *n_items) return;
+  const MoeItem it = moe_item(items, blockIdx.y);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int lt0 = blockIdx.x * TN;  // first output tile within the expert
+  const uint32_t nch = static_cast<uint32_t>(nchunks);
+  const uint32_t n_params = static_cast<uint32_t>(ntiles) * nch * nbc * 16;
+  const auto a_rsrc = buffer_rsrc(A, static_cast<uint32_t>(a_rows) * lda * 2);
+  __amdgpu_buffer_rsrc_t q_rsrc[NV], s_rsrc[NV], z_rsrc[NV];
+  uint32_t tile[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const bool second = EPI == EPI_GLU && (v & 1);
+    q_rsrc[v] = buffer_rsrc(second ? qt2 : qt, static_cast<uint32_t>(ntiles) * nch * 1024);
+    s_rsrc[v] = buffer_rsrc(second ? sc2 : sc, n_params * 2);
+    z_rsrc[v] = buffer_rsrc(second ? zp2 : zp, HAS_ZP ? zp_byte<BITS>(n_params) : 0u);
+    // Output tiles past the expert's last read its last one and store nothing.
+    const int lt = min(lt0 + (EPI == EPI_GLU ? v / 2 : v), out_tiles - 1);
+    tile[v] = static_cast<uint32_t>(it.e * tiles_per_expert + lt + (second ? tile_off2 : 0));
+  }
+  struct Weights {
+    uint4_t w[NV];
+    uint32_t s[NV][NJ], z[NV][NJ];
+  };
+  struct Rows {
+    uint4_t a[STEPS];
+  };
+  auto load_w = [&](uint32_t c, Weights& st) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      st.w[v] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc[v], (tile[v] * nch * 64 + lane) * 16, c * 1024, 0);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const uint32_t e = ((tile[v] * nch + c) * nbc + ((SPLIT ? 32 * j + 8 * g : g * GW) >> bsc_shift)) * 16 + r;
+        st.s[v][j] = __builtin_amdgcn_raw_buffer_load_b16(s_rsrc[v], e * 2, 0, 0);
+        if constexpr (HAS_ZP) st.z[v][j] = __builtin_amdgcn_raw_buffer_load_b8(z_rsrc[v], zp_byte<BITS>(e), 0, 0);
+      }
+    }
+  };
+  Weights wa, wb;
+  Rows ra, rb;
+  if (static_cast<uint32_t>(wave) < nch) load_w(wave, wa);  // needs the item only; the rows' index comes meanwhile
+  const int src = r < it.rows ? (perm ? perm[it.row0 + r] / perm_div : it.row0 + r) : -1;
+  const uint32_t a_row = src >= 0 ? static_cast<uint32_t>(src) * lda * 2 : 0x80000000u;
+  auto load_a = [&](uint32_t c, Rows& st) {
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      const uint32_t k = c * CW + 32 * i + 8 * g;  // lda = K, a multiple of 8: a step lies wholly in or past K
+      st.a[i] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, k < static_cast<uint32_t>(lda) ? a_row + k * 2 : 0x80000000u, 0, 0);
+    }
+  };
+  float4_t acc[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) acc[v] = float4_t{0.f, 0.f, 0.f, 0.f};
+  const uint32_t zsh = zp_shift<BITS>(r);
+  auto compute = [&](const Weights& st, const Rows& rows) {
+    uint4_t wn[NV];
+    uint32_t par[NV][STEPS];  // scale | (1024 + zero as f16) << 16 of the lane's weights in each step
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      wn[v] = natural_words<BITS>(st.w[v]);
+      uint32_t own[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        own[j] = HAS_ZP ? (st.s[v][j] & 0xFFFFu) | ((0x6400u + zp_field<BITS>(st.z[v][j], zsh)) << 16) : st.s[v][j];
+      if constexpr (SPLIT) {
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) par[v][i] = own[i];
+      } else {
+        natural_params<BITS>(own[0], par[v]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        // (unpack_step reads the low halves of its parameters.)
+        const uint32_t zz = HAS_ZP ? par[v][i] >> 16 : 0x6400u + (1u << (BITS - 1));
+        const half8_t b = unpack_step<BITS>(wn[v], i, __builtin_bit_cast(half2_t, zz), __builtin_bit_cast(half2_t, par[v][i]));
+        acc[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, __builtin_bit_cast(half8_t, rows.a[i]), acc[v], 0, 0, 0);
+      }
+  };
+  if (static_cast<uint32_t>(wave) < nch) {
+    load_a(wave, ra);
+    for (uint32_t c = wave;;) {
+      const bool second = c + NW < nch;
+      if (second) {
+        load_w(c + NW, wb);
+        load_a(c + NW, rb);
+      }
+      compute(wa, ra);
+      if (!second) break;
+      const bool third = c + 2 * NW < nch;
+      if (third) {
+        load_w(c + 2 * NW, wa);
+        load_a(c + 2 * NW, ra);
+      }
+      compute(wb, rb);
+      if (!third) break;
+      c += 2 * NW;
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v) red[(wave * NV + v) * 64 + lane] = acc[v];
+  __syncthreads();
+  // The output tiles go to the wavefronts in turn: lane (16g + r) holds row r, columns 4g .. 4g + 3.
+#pragma unroll
+  for (int t0 = 0; t0 < TN; t0 += NW) {
+    const int tn = t0 + wave;
+    if (tn >= TN) return;
+    if (r >= it.rows || lt0 + tn >= out_tiles) continue;
+    auto total = [&](int v) {
+      float4_t part[NW];
+#pragma unroll
+      for (int w2 = 0; w2 < NW; ++w2) part[w2] = red[(w2 * NV + v) * 64 + lane];
+      float4_t t = part[0];
+#pragma unroll
+      for (int w2 = 1; w2 < NW; ++w2) t += part[w2];
+      return t;
+    };
+    const float4_t s1 = total(EPI == EPI_GLU ? 2 * tn : tn);
+    float4_t s2{};
+    if constexpr (EPI == EPI_GLU) s2 = total(2 * tn + 1);
+    const int n = (lt0 + tn) * 16 + 4 * g;
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float h = rt<DT_F16>(s1[e]);
+      if (EPI != EPI_STORE && bias1)
+        h = rt<DT_F16>(h + load_float_rt(bias1, bias_dt, static_cast<int64_t>(it.e) * bias_ld + n + e));
+      float l = 0.f;
+      if constexpr (EPI == EPI_GLU) {
+        l = rt<DT_F16>(s2[e]);
+        if (bias2)
+          l = rt<DT_F16>(l + load_float_rt(bias2, bias_dt, static_cast<int64_t>(it.e) * bias_ld + n + e + tile_off2 * 16));
+      }
+      y[e] = EPI == EPI_STORE ? h : activate<DT_F16>(act, h, l, alpha, beta, limit);
+    }
+    const half2_t lo = {static_cast<_Float16>(y[0]), static_cast<_Float16>(y[1])};
+    const half2_t hi = {static_cast<_Float16>(y[2]), static_cast<_Float16>(y[3])};
+    const int orow = out_perm ? out_perm[it.row0 + r] : it.row0 + r;
+    *reinterpret_cast<uint2*>(out + static_cast<int64_t>(orow) * ldo + n) =
+        make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+  }
 }
 
 // The same product for any float types (A in a_dt, weights dequantized in WDT, out in out_dt):
@@ -556,14 +733,14 @@ template <int BITS, int WDT, int ZK>
 __global__ __launch_bounds__(256) void k_moe_gemm_general(
     const uint4_t* __restrict__ qt, const void* __restrict__ sc, const void* __restrict__ zp, int nchunks, int nbc,
     int bsc_shift, int tiles_per_expert, int K, const void* __restrict__ A, int a_dt, int lda,
-    const int* __restrict__ perm, int perm_div, const int* __restrict__ items, const int* __restrict__ n_items,
-    const int* __restrict__ offsets, const int* __restrict__ counts, void* __restrict__ out, int out_dt, int ldo) {
+    const int* __restrict__ perm, int perm_div, const int4* __restrict__ items, const int* __restrict__ n_items,
+    void* __restrict__ out, int out_dt, int ldo) {
   constexpr int CW = 512 / BITS;
   constexpr int GW = CW / 4;
   constexpr int PER_WORD = 32 / BITS;
   __shared__ float red[4][kMoeRows][16];
   if (static_cast<int>(blockIdx.y) >= *n_items) return;
-  const MoeItem it = moe_item(items, blockIdx.y, offsets, counts, kMoeRows);
+  const MoeItem it = moe_item(items, blockIdx.y);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
   const int64_t t = static_cast<int64_t>(it.e) * tiles_per_expert + blockIdx.x;
@@ -777,14 +954,14 @@ struct MoeEpilogue {
   const void *bias1 = nullptr, *bias2 = nullptr;
   int bias_dt = TMH_F32, bias_ld = 0, act = ACT_IDENTITY;
   float alpha = 1.f, beta = 0.f, limit = 0.f;
-  int rows = 32;                   // rows per work item: 32 or 64
+  int rows = 32;                   // rows per work item: 32 or 64 (k_moe_rows: 16)
+  bool few_rows = false;           // the product for items of few rows, k_moe_rows
   const int* out_perm = nullptr;   // output row of each sorted row (else the sorted row itself)
 };
 
 template <int BITS, bool HAS_ZP, bool SPLIT, int EPI, int MT>
 void launch_moe_f16_e(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
-                      const int* items, const int* n_items, int max_items, const int* offsets, const int* counts,
-                      void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
+                      const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
   const tmh_weight* w2 = ep.w2 ? ep.w2 : w;
   // Groups of eight output tiles per workgroup, one after the other: the stored products (fc2,
   // many groups per item) run four, so the workgroups' prologues and the last partial round of
@@ -798,7 +975,7 @@ void launch_moe_f16_e(const tmh_weight* w, int tpe, const void* A, int a_rows, i
       static_cast<const uint8_t*>(w->d_zero), reinterpret_cast<const uint4_t*>(w2->d_q),                              \
       static_cast<const uint16_t*>(w2->d_scale), static_cast<const uint8_t*>(w2->d_zero), ep.tile_off2,               \
       static_cast<int>(w->ntiles), static_cast<int>(w->nchunks), w->nbc, bsc_shift_moe(w), tpe, ep.out_tiles, gpw,    \
-      static_cast<const _Float16*>(A), a_rows, lda, perm, perm_div, items, n_items, offsets, counts, ep.bias1,        \
+      static_cast<const _Float16*>(A), a_rows, lda, perm, perm_div, items, n_items, ep.bias1,        \
       ep.bias2, ep.bias_dt, ep.bias_ld, ep.act, ep.alpha, ep.beta, ep.limit, static_cast<_Float16*>(out), ldo,       \
       ep.out_perm
   if (uint32_t* tl = timeline_slots(TMH_TL_MOE_GEMM, static_cast<int64_t>(grid.x) * grid.y * 8))
@@ -808,12 +985,53 @@ void launch_moe_f16_e(const tmh_weight* w, int tpe, const void* A, int a_rows, i
 #undef TMH_MOE_ARGS
 }
 
+template <int BITS, bool HAS_ZP, bool SPLIT, int EPI, int TN, int NW>
+void go_moe_rows(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
+                 const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep,
+                 hipStream_t s) {
+  const tmh_weight* w2 = ep.w2 ? ep.w2 : w;
+  const dim3 grid(static_cast<unsigned>((ep.out_tiles + TN - 1) / TN), static_cast<unsigned>(max_items));
+  k_moe_rows<BITS, HAS_ZP, SPLIT, EPI, TN, NW><<<grid, 64 * NW, 0, s>>>(
+      reinterpret_cast<const uint4_t*>(w->d_q), static_cast<const uint16_t*>(w->d_scale),
+      static_cast<const uint8_t*>(w->d_zero), reinterpret_cast<const uint4_t*>(w2->d_q),
+      static_cast<const uint16_t*>(w2->d_scale), static_cast<const uint8_t*>(w2->d_zero), ep.tile_off2,
+      static_cast<int>(w->ntiles), static_cast<int>(w->nchunks), w->nbc, bsc_shift_moe(w), tpe, ep.out_tiles,
+      static_cast<const _Float16*>(A), a_rows, lda, perm, perm_div, items, n_items, ep.bias1, ep.bias2, ep.bias_dt,
+      ep.bias_ld, ep.act, ep.alpha, ep.beta, ep.limit, static_cast<_Float16*>(out), ldo, ep.out_perm);
+}
+
+template <int BITS, bool HAS_ZP, bool SPLIT, int EPI>
+void launch_moe_rows_e(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
+                       const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep,
+                       hipStream_t s) {
+  // One output tile (of both weights) over four wavefronts for swiglu; else two tiles, over two
+  // wavefronts where K is short (8 tokens of 128 experts, fc1 and fc3 with 16 chunks: 1,4 47.7 us a
+  // call, 1,2 47.9, 1,8 52.3, 2,4 50.2; fc2 with 6: 2,2 47.6, 1,2 48.1, 2,4 49.1, 4,2 50.5).
+  if constexpr (EPI == EPI_GLU)
+    go_moe_rows<BITS, HAS_ZP, SPLIT, EPI, 1, 4>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s);
+  else if (w->nchunks <= 8)
+    go_moe_rows<BITS, HAS_ZP, SPLIT, EPI, 2, 2>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s);
+  else
+    go_moe_rows<BITS, HAS_ZP, SPLIT, EPI, 2, 4>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s);
+}
+
+template <int BITS, bool HAS_ZP, bool SPLIT>
+void launch_moe_rows(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
+                     const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep,
+                     hipStream_t s) {
+#define TMH_MOE_ROWS(E) \
+  launch_moe_rows_e<BITS, HAS_ZP, SPLIT, E>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s)
+  if (ep.kind == EPI_GLU) TMH_MOE_ROWS(EPI_GLU);
+  else if (ep.kind == EPI_ACT) TMH_MOE_ROWS(EPI_ACT);
+  else TMH_MOE_ROWS(EPI_STORE);
+#undef TMH_MOE_ROWS
+}
+
 template <int BITS, bool HAS_ZP, bool SPLIT>
 void launch_moe_f16_v(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
-                      const int* items, const int* n_items, int max_items, const int* offsets, const int* counts,
-                      void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
+                      const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
 #define TMH_MOE_EPI(E, MT) \
-  launch_moe_f16_e<BITS, HAS_ZP, SPLIT, E, MT>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, offsets, counts, out, ldo, ep, s)
+  launch_moe_f16_e<BITS, HAS_ZP, SPLIT, E, MT>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s)
   if (ep.rows == 64) {
     if (ep.kind == EPI_GLU) TMH_MOE_EPI(EPI_GLU, 4);
     else if (ep.kind == EPI_ACT) TMH_MOE_EPI(EPI_ACT, 4);
@@ -828,12 +1046,22 @@ void launch_moe_f16_v(const tmh_weight* w, int tpe, const void* A, int a_rows, i
 
 template <int BITS>
 void launch_moe_f16(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
-                    const int* items, const int* n_items, int max_items, const int* offsets, const int* counts,
-                    void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
+                    const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
   const bool zp = w->zp_kind == TMH_ZP_PACKED;
   const bool split = w->block_size < (512 / BITS) / 4;
+  if constexpr (BITS != 2) {
+    if (ep.few_rows) {
+#define TMH_MOE_FEW(Z, S) launch_moe_rows<BITS, Z, S>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s)
+      if (zp && split) TMH_MOE_FEW(true, true);
+      else if (zp) TMH_MOE_FEW(true, false);
+      else if (split) TMH_MOE_FEW(false, true);
+      else TMH_MOE_FEW(false, false);
+#undef TMH_MOE_FEW
+      return;
+    }
+  }
 #define TMH_MOE_F16(Z, S) \
-  launch_moe_f16_v<BITS, Z, S>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, offsets, counts, out, ldo, ep, s)
+  launch_moe_f16_v<BITS, Z, S>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s)
   if (zp && split) TMH_MOE_F16(true, true);
   else if (zp) TMH_MOE_F16(true, false);
   else if (split) TMH_MOE_F16(false, true);
@@ -843,37 +1071,32 @@ void launch_moe_f16(const tmh_weight* w, int tpe, const void* A, int a_rows, int
 
 template <int BITS, int WDT>
 void launch_moe_general_w(const tmh_weight* w, int tpe, const void* A, int a_dt, int lda, const int* perm, int perm_div,
-                          const int* items, const int* n_items, int max_items, const int* offsets, const int* counts,
-                          void* out, int out_dt, int ldo, hipStream_t s) {
+                          const int4* items, const int* n_items, int max_items, void* out, int out_dt, int ldo, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(tpe), static_cast<unsigned>(max_items));
   const auto* qt = reinterpret_cast<const uint4_t*>(w->d_q);
   const int sh = bsc_shift_moe(w);
   if (w->zp_kind == TMH_ZP_PACKED)
     k_moe_gemm_general<BITS, WDT, TMH_ZP_PACKED><<<grid, 256, 0, s>>>(
         qt, w->d_scale, w->d_zero, static_cast<int>(w->nchunks), w->nbc, sh, tpe, static_cast<int>(w->K), A, a_dt, lda,
-        perm, perm_div, items, n_items, offsets, counts, out, out_dt, ldo);
+        perm, perm_div, items, n_items, out, out_dt, ldo);
   else
     k_moe_gemm_general<BITS, WDT, TMH_ZP_NONE><<<grid, 256, 0, s>>>(
         qt, w->d_scale, w->d_zero, static_cast<int>(w->nchunks), w->nbc, sh, tpe, static_cast<int>(w->K), A, a_dt, lda,
-        perm, perm_div, items, n_items, offsets, counts, out, out_dt, ldo);
+        perm, perm_div, items, n_items, out, out_dt, ldo);
 }
 
 template <int BITS>
 void launch_moe_general(const tmh_weight* w, int tpe, const void* A, int a_dt, int lda, const int* perm, int perm_div,
-                        const int* items, const int* n_items, int max_items, const int* offsets, const int* counts,
-                        void* out, int out_dt, int ldo, hipStream_t s) {
+                        const int4* items, const int* n_items, int max_items, void* out, int out_dt, int ldo, hipStream_t s) {
   switch (w->wdtype) {
     case TMH_F16:
-      launch_moe_general_w<BITS, DT_F16>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, offsets,
-                                         counts, out, out_dt, ldo, s);
+      launch_moe_general_w<BITS, DT_F16>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, out_dt, ldo, s);
       break;
     case TMH_BF16:
-      launch_moe_general_w<BITS, DT_BF16>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, offsets,
-                                          counts, out, out_dt, ldo, s);
+      launch_moe_general_w<BITS, DT_BF16>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, out_dt, ldo, s);
       break;
     default:
-      launch_moe_general_w<BITS, DT_F32>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, offsets,
-                                         counts, out, out_dt, ldo, s);
+      launch_moe_general_w<BITS, DT_F32>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, out_dt, ldo, s);
   }
 }
 
@@ -888,22 +1111,21 @@ bool moe_fast(const tmh_weight* w, int a_dt, const void* A, int a_rows, int lda)
 // One grouped product: rows (gathered through perm when given) times each row's expert. The
 // fast path applies the epilogue; the general path stores the sums (EPI_STORE only).
 void moe_gemm(const tmh_weight* w, int experts, const void* A, int a_dt, int a_rows, int lda, const int* perm,
-              int perm_div, const int* items, const int* n_items, int max_items, const int* offsets,
-              const int* counts, void* out, int ldo, hipStream_t s, MoeEpilogue ep = MoeEpilogue()) {
+              int perm_div, const int4* items, const int* n_items, int max_items, void* out, int ldo, hipStream_t s, MoeEpilogue ep = MoeEpilogue()) {
   const int tpe = static_cast<int>(w->N / experts / 16);
   if (moe_fast(w, a_dt, A, a_rows, lda)) {
     if (ep.out_tiles == 0) ep.out_tiles = tpe;
     switch (w->bits) {
-      case 2: launch_moe_f16<2>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, offsets, counts, out, ldo, ep, s); break;
-      case 4: launch_moe_f16<4>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, offsets, counts, out, ldo, ep, s); break;
-      default: launch_moe_f16<8>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, offsets, counts, out, ldo, ep, s);
+      case 2: launch_moe_f16<2>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s); break;
+      case 4: launch_moe_f16<4>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s); break;
+      default: launch_moe_f16<8>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s);
     }
     return;
   }
   switch (w->bits) {
-    case 2: launch_moe_general<2>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, offsets, counts, out, a_dt, ldo, s); break;
-    case 4: launch_moe_general<4>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, offsets, counts, out, a_dt, ldo, s); break;
-    default: launch_moe_general<8>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, offsets, counts, out, a_dt, ldo, s);
+    case 2: launch_moe_general<2>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, a_dt, ldo, s); break;
+    case 4: launch_moe_general<4>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, a_dt, ldo, s); break;
+    default: launch_moe_general<8>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, a_dt, ldo, s);
   }
 }
 
@@ -1040,26 +1262,33 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
                         (!two || moe_fast(fc3, x_dtype, d_x, static_cast<int>(T), static_cast<int>(H))) &&
                         fc2->wdtype == TMH_F16 && fc2->zp_kind != TMH_ZP_FLOAT && inter_i % 8 == 0 &&
                         tk * inter_i * 2 < (int64_t(1) << 31) && (fc2->ntiles + 1) * fc2->nchunks * 1024 < (int64_t(1) << 31);
-  const int rows = all_fast && tk > 24 * E ? 64 : kMoeRows;
-  const int max_items = static_cast<int>((tk + rows - 1) / rows + E);
+  // Few rows an expert and few experts reached (at most min(E, T k)): k_moe_rows, items of 16 rows.
+  // Where more experts are reached the product that walks K reads as fast with less instruction work,
+  // from fewer experts on the narrower they are (q4, us per call, this product / moe_gemm_f16, 2 to 8
+  // rows an expert: 2048/768 with 32 experts 31.5-35.4 / 41.5-43.7, 64 experts 51.0-59.6 / 60.2-63.4,
+  // 128 experts 85.9-98.3 / 86.1-90.5; 1024/512 with 32 experts 22.4-24.7 / 24.4-26.4, 64 experts
+  // 29.3-32.4 / 27.8-29.5).
+  const bool few = all_fast && fc1->bits != 2 && fc2->bits != 2 && (!two || fc3->bits != 2) && tk <= 8 * E &&
+                   std::min(E, tk) <= (fc1->nchunks >= 16 ? 64 : 32);
+  const int rows = few ? 16 : all_fast && tk > 24 * E ? 64 : kMoeRows;
+  // An item is the last of its expert (at most one an expert, and one a routed row) or full.
+  const int max_items = static_cast<int>(tk / rows + std::min(E, tk));
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
     off += align256(bytes);
     return at;
   };
-  const size_t o_counts = take(E * 4), o_offsets = take(E * 4), o_nitems = take(4);
-  const size_t o_items = take(static_cast<size_t>(max_items) * 4), o_topi = take(tk * 4), o_topw = take(tk * 4);
+  const size_t o_nitems = take(4);
+  const size_t o_items = take(static_cast<size_t>(max_items) * sizeof(int4)), o_topi = take(tk * 4), o_topw = take(tk * 4);
   const size_t o_perm = take(tk * 4), o_slot = take(tk * 4);
   const size_t o_h1 = take(tk * n1 * es), o_h3 = two ? take(tk * n1 * es) : 0;
   const size_t o_act = take(tk * inter * es), o_o = take(tk * H * es);
   auto* ws = static_cast<uint8_t*>(workspace(ctx, off, s));
   if (!ws)
     return fail(ctx, TMH_ERR_UNSUPPORTED, "QMoE needs a %zu-byte workspace; run it once outside graph capture first", off);
-  auto* counts = reinterpret_cast<int*>(ws + o_counts);
-  auto* offsets = reinterpret_cast<int*>(ws + o_offsets);
   auto* n_items = reinterpret_cast<int*>(ws + o_nitems);
-  auto* items = reinterpret_cast<int*>(ws + o_items);
+  auto* items = reinterpret_cast<int4*>(ws + o_items);
   auto* topi = reinterpret_cast<int*>(ws + o_topi);
   auto* topw = reinterpret_cast<float*>(ws + o_topw);
   auto* perm = reinterpret_cast<int*>(ws + o_perm);
@@ -1070,7 +1299,21 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
   void* o = ws + o_o;
   const int ti = static_cast<int>(T), ki = k, ei = static_cast<int>(E), tki = static_cast<int>(tk);
   const unsigned route_grid = static_cast<unsigned>((T + 3) / 4);
-  {
+  if (T <= kFusedRouteTokens && !ctx->tl) {  // (a timeline records the two kernels)
+#define TMH_MOE_RP_J(RDT, EJ) \
+  k_moe_route_plan<RDT, EJ><<<1, 1024, 0, s>>>(d_router, ti, ei, ki, rows, topi, topw, items, n_items, perm, slot_pos)
+#define TMH_MOE_RP(RDT)                 \
+  if (ei <= 128) TMH_MOE_RP_J(RDT, 2);  \
+  else if (ei <= 256) TMH_MOE_RP_J(RDT, 4); \
+  else TMH_MOE_RP_J(RDT, 16)
+    switch (router_dtype) {
+      case TMH_F16: TMH_MOE_RP(DT_F16); break;
+      case TMH_BF16: TMH_MOE_RP(DT_BF16); break;
+      default: TMH_MOE_RP(DT_F32);
+    }
+#undef TMH_MOE_RP
+#undef TMH_MOE_RP_J
+  } else {
     // Router keys per lane: 2 up to 128 experts, 4 up to 256, 16 up to 1024.
     uint32_t* tl = timeline_slots(TMH_TL_MOE_ROUTE, static_cast<int64_t>(route_grid) * 4);
 #define TMH_MOE_ROUTE_J(RDT, EJ)                                                                              \
@@ -1087,11 +1330,11 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
     }
 #undef TMH_MOE_ROUTE
 #undef TMH_MOE_ROUTE_J
+    if (uint32_t* tl = timeline_slots(TMH_TL_MOE_PLAN, 16))
+      k_moe_plan_tl<<<1, 1024, 0, s>>>(ei, rows, topi, tki, items, n_items, perm, slot_pos, tl);
+    else
+      k_moe_plan<<<1, 1024, 0, s>>>(ei, rows, topi, tki, items, n_items, perm, slot_pos);
   }
-  if (uint32_t* tl = timeline_slots(TMH_TL_MOE_PLAN, 16))
-    k_moe_plan_tl<<<1, 1024, 0, s>>>(counts, ei, rows, topi, tki, offsets, items, n_items, perm, slot_pos, tl);
-  else
-    k_moe_plan<<<1, 1024, 0, s>>>(counts, ei, rows, topi, tki, offsets, items, n_items, perm, slot_pos);
   TMH_TRY(check_launch(ctx, "k_moe_plan"));
   const int hi = static_cast<int>(H), n1i = static_cast<int>(n1), inti = static_cast<int>(inter);
   // fc1 (and fc3) with the activation in the product's epilogue where the fast path allows it:
@@ -1099,6 +1342,7 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
   // Interleaved swiglu pairs and the general path store the sums and activate separately.
   MoeEpilogue ep;
   ep.rows = rows;
+  ep.few_rows = few;
   ep.bias1 = d_fc1_bias;
   ep.bias_dt = bias_dtype;
   ep.bias_ld = n1i;
@@ -1123,11 +1367,11 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
     } else {
       ep.kind = EPI_ACT;
     }
-    moe_gemm(fc1, ei, d_x, x_dtype, ti, hi, perm, ki, items, n_items, max_items, offsets, counts, hact, inti, s, ep);
+    moe_gemm(fc1, ei, d_x, x_dtype, ti, hi, perm, ki, items, n_items, max_items, hact, inti, s, ep);
     TMH_TRY(check_launch(ctx, "k_moe_gemm (fc1)"));
   } else {
-    moe_gemm(fc1, ei, d_x, x_dtype, ti, hi, perm, ki, items, n_items, max_items, offsets, counts, h1, n1i, s);
-    if (two) moe_gemm(fc3, ei, d_x, x_dtype, ti, hi, perm, ki, items, n_items, max_items, offsets, counts, h3, n1i, s);
+    moe_gemm(fc1, ei, d_x, x_dtype, ti, hi, perm, ki, items, n_items, max_items, h1, n1i, s);
+    if (two) moe_gemm(fc3, ei, d_x, x_dtype, ti, hi, perm, ki, items, n_items, max_items, h3, n1i, s);
     TMH_TRY(check_launch(ctx, "k_moe_gemm (fc1)"));
     const int64_t act_n = tk * (activation == ACT_SWIGLU ? inter : n1);
     const unsigned act_grid = static_cast<unsigned>((act_n + 255) / 256);
@@ -1147,9 +1391,10 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
   const bool fc2_fast = moe_fast(fc2, x_dtype, hact, tki, inti);
   MoeEpilogue ep2;
   ep2.rows = rows;
+  ep2.few_rows = few;
   ep2.out_perm = fc2_fast ? perm : nullptr;
   const int* o_rows = fc2_fast ? nullptr : slot_pos;
-  moe_gemm(fc2, ei, hact, x_dtype, tki, inti, nullptr, 1, items, n_items, max_items, offsets, counts, o, hi, s, ep2);
+  moe_gemm(fc2, ei, hact, x_dtype, tki, inti, nullptr, 1, items, n_items, max_items, o, hi, s, ep2);
   TMH_TRY(check_launch(ctx, "k_moe_gemm (fc2)"));
   // H is a multiple of 16: eight columns per thread.
   const unsigned out_grid = static_cast<unsigned>((T * H / 8 + 255) / 256);
