@@ -95,7 +95,8 @@ class Timeline:
             start, end = int(t0.min()), int(t1.max())
             out.append({"kernel": kernel, "waves": int(ok.sum()), "start_us": start * TICK_US,
                         "end_us": end * TICK_US, "us": (end - start) * TICK_US,
-                        "ghz": float(cyc.sum()) / float(real.sum()) / 10.0 if real.sum() else None})
+                        # (Wavefronts of a few ticks, an empty kernel's, tell no rate: each end is a tick off.)
+                        "ghz": float(cyc.sum()) / float(real.sum()) / 10.0 if real.sum() >= 16 * len(real) else None})
         return out
 
     def free(self) -> None:
