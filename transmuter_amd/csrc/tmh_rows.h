@@ -117,7 +117,9 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
   const uint32_t n_params = ntiles * nch * nbc * 16;
   const bool a_f32 = OP == ROW_INT || (OP == ROW_GEN && (types >> 24) == DT_F32);
   const uint32_t a_size = a_f32 ? 4 : 2;
-  const uint32_t zk = kinds & 0xFFu;
+  // Without zero points zp is null; ROW_GEN's kinds, which tells float ones, is no preloaded argument,
+  // and waiting for it ahead of the first loads would cost every launch of the other paths.
+  const uint32_t zk = OP == ROW_GEN ? kinds & 0xFFu : zp ? TMH_ZP_PACKED : TMH_ZP_NONE;
   const bool s_f32 = OP == ROW_INT || (OP == ROW_GEN && ((kinds >> 8) & 0xFFu) == DT_F32);
   const auto q_rsrc = buffer_rsrc(qt, ntiles * nch * 1024);
   const auto s_rsrc = buffer_rsrc(sc, n_params * (s_f32 ? 4 : 2));
