@@ -9,6 +9,7 @@
 //   sum_k (a - az_m)(b - bz_n) = sum_k sa sb + cb_n * rs_m + ca_m * cs_n + K * ca_m * cb_n (mod 2^32)
 // with ca_m = oa - az_m, cb_n = ob - bz_n, rs_m = sum_k sa = (sum_k a) - oa K, cs_n = sum_k sb.
 #include <algorithm>
+#include <type_traits>
 
 #include "tmh_device.h"
 #include "tmh_internal.h"
@@ -19,6 +20,7 @@ struct tmh_int8_weight {
   int8_t* d_bt = nullptr;        // [N][Kp] s8, zero past K
   int32_t* d_cs = nullptr;       // [N] column sums of sb over k < K
   int32_t* d_cb = nullptr;       // [N] ob - bz_n
+  bool symmetric = false;        // s8 B without zero points: every ob - bz_n is 0
   size_t device_bytes = 0;
 };
 
@@ -118,16 +120,10 @@ __global__ __launch_bounds__(256) void k_i8_colsum(const uint32_t* __restrict__ 
   cb[n] = (b_signed ? 0 : 128) - bz;
 }
 
-// At most n vector-memory operations of this thread outstanding (n a multiple of 4, up to 12).
-__device__ __forceinline__ void wait_vm(uint32_t n) {
-  if (n >= 12)
-    __builtin_amdgcn_s_waitcnt(12 | (7 << 4) | (15 << 8));
-  else if (n >= 8)
-    __builtin_amdgcn_s_waitcnt(8 | (7 << 4) | (15 << 8));
-  else if (n >= 4)
-    __builtin_amdgcn_s_waitcnt(4 | (7 << 4) | (15 << 8));
-  else
-    __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+// At most N vector-memory operations of this thread outstanding (N below 16), and no LDS operation.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  __builtin_amdgcn_s_waitcnt(N | (7 << 4));
 }
 
 // 128 x 128 outputs per workgroup of eight wavefronts: wavefront w computes the 64 x 64 quadrant
@@ -135,14 +131,18 @@ __device__ __forceinline__ void wait_vm(uint32_t n) {
 // so a lane ends with 4 consecutive columns of one row); the halves add through LDS at the end.
 // Each step's A rows and Bt rows (KQ bytes of k) go global -> LDS by buffer_load ... lds, 16 bytes
 // per lane into rows whose 16-byte pieces are XOR-swizzled by row (frag_swizzle: conflict-free
-// fragment reads; a lane loads the global piece that belongs in its slot), issued STAGES - 1 steps
-// ahead into a ring of STAGES stages, so one barrier per step both publishes step s and frees the
-// stage that the next issue overwrites.
+// fragment reads; a lane loads the global piece that belongs in its slot), issued three steps ahead
+// into a ring of four stages, and the fragments of step s + 1 are read while step s multiplies, so one
+// barrier per step both publishes stage s + 1 and frees the stage that the next issue overwrites.
+// A step is bound by instruction issue: its 16 MFMAs a wavefront take 256 cycles, each vector
+// instruction beside them 4, on SIMDs that two wavefronts share. So the offsets along k are scalar, a
+// stage's address costs two additions, and A's row sums are only taken for a B that needs them. 2048^3
+// u8 x s8 without zero points 19.2 -> 16.4 us (1050 TOP/s), 4096^3 100 -> 84; u8 x u8 19.1 -> 18.4.
+// Removing alone the loads, the fragment reads or the products from a step left 88-94% of its time.
 // A: rows past M lie past the buffer range and read zeros (their outputs are not stored), pieces
 // past K are pointed past it too (K is a multiple of 16). The raw bytes of A are summed per row
-// (v_dot4_u32_u8; v_dot4_i32_i8 for s8 A) as the fragments are read, by the wavefronts of the left
-// quadrants.
-template <bool A_SIGNED, int KQ, int STAGES, int NW = 8>
+// (v_dot4_u32_u8; v_dot4_i32_i8 for s8 A) as they multiply (ROW_SUMS).
+template <bool A_SIGNED, bool ROW_SUMS, int KQ, int STAGES, int NW = 8>
 __global__ __launch_bounds__(64 * NW) void k_mmi_bt(const uint8_t* __restrict__ a,
                                                 const int8_t* __restrict__ bt, const int32_t* __restrict__ cs,
                                                 const int32_t* __restrict__ cb, const uint8_t* __restrict__ a_zero,
@@ -153,8 +153,7 @@ __global__ __launch_bounds__(64 * NW) void k_mmi_bt(const uint8_t* __restrict__ 
   constexpr int KS = NW / 4;                    // wavefronts sharing a quadrant, each a k-part of a step
   constexpr int DMA = kQT / RPI / NW;           // DMA instructions per wavefront per operand and step
   constexpr int STAGE = 2 * kQT * KQ;           // bytes of one stage (A and B tiles)
-  constexpr int SUB = KQ / KS / 64;             // MFMA k-steps of 64 in a wavefront's k-part
-  static_assert(DMA >= 1 && SUB >= 1, "step shape");
+  static_assert(DMA >= 1 && KQ / KS == 64 && 2 * KQ <= kQPad && STAGES == 4, "step shape");
   constexpr uint32_t aflip = A_SIGNED ? 0u : 0x80808080u;
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -174,7 +173,8 @@ __global__ __launch_bounds__(64 * NW) void k_mmi_bt(const uint8_t* __restrict__ 
   const uint8_t* a8 = a + static_cast<int64_t>(blockIdx.z) * M * K;
   const auto a_rsrc = buffer_rsrc(a8, M * K);
   const auto b_rsrc = buffer_rsrc(bt, N * Kp);
-  // This lane's DMA rows (RPI-row groups DMA * w + j) and the global piece its slot holds.
+  // This lane's DMA rows (RPI-row groups DMA * w + j) and the global piece its slot holds: the step's
+  // offset along k goes to the loads' scalar offset, so a step's loads cost no vector instruction.
   uint32_t a_off[DMA], b_off[DMA], gpc[DMA];
 #pragma unroll
   for (int j = 0; j < DMA; ++j) {
@@ -188,11 +188,22 @@ __global__ __launch_bounds__(64 * NW) void k_mmi_bt(const uint8_t* __restrict__ 
     uint8_t* sa = lds + (s % STAGES) * STAGE;
     uint8_t* sb = sa + kQT * KQ;
     const uint32_t k0 = s * KQ;
+    if (k0 + KQ <= K) {
 #pragma unroll
-    for (int j = 0; j < DMA; ++j) {
-      const int row0 = RPI * (DMA * wave + j);
-      lds_dma16(a_rsrc, sa + row0 * KQ, k0 + gpc[j] * 16 < K ? a_off[j] + k0 : 0x80000000u, 0);
-      lds_dma16(b_rsrc, sb + row0 * KQ, b_off[j] + k0, 0);
+      for (int j = 0; j < DMA; ++j) {
+        const int row0 = RPI * (DMA * wave + j);
+        // Rows past M: their offset is past the range by itself (the range check leaves the scalar
+        // offset out, and (m0 + row) * K is at least M * K).
+        lds_dma16(a_rsrc, sa + row0 * KQ, a_off[j], k0);
+        lds_dma16(b_rsrc, sb + row0 * KQ, b_off[j], k0);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < DMA; ++j) {
+        const int row0 = RPI * (DMA * wave + j);
+        lds_dma16(a_rsrc, sa + row0 * KQ, k0 + gpc[j] * 16 < K ? a_off[j] + k0 : 0x80000000u, 0);
+        lds_dma16(b_rsrc, sb + row0 * KQ, b_off[j], k0);
+      }
     }
   };
   int4_t acc[4][4];
@@ -201,58 +212,98 @@ __global__ __launch_bounds__(64 * NW) void k_mmi_bt(const uint8_t* __restrict__ 
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = int4_t{0, 0, 0, 0};
   uint32_t raw[4] = {0u, 0u, 0u, 0u};
+  // Fragments of one step: 64 bytes of k of the quadrant's 64 rows of A and of B^T.
+  struct Frags {
+    uint4_t a[4];
+    int4_t b[4];
+  };
+  // This lane's 16-byte piece of the fragments' first rows: the same slot in every 16th row. Steps go in
+  // pairs, so a stage is a scalar (its pair) and a constant (its parity) away.
+  const int slot = ((kh * (PPR / KS) + g) ^ frag_swizzle<PPR>(r)) << 4;
+  const uint32_t lane_a = (64 * wm + r) * KQ + slot, lane_b = kQT * KQ + (64 * wn + r) * KQ + slot;
+  auto read = [&](uint32_t s, auto odd, Frags& f) {
+    const uint32_t pair = (s & 2) ? 2 * STAGE : 0;
+    const uint8_t* pa = lds + (lane_a + pair);
+    const uint8_t* pb = lds + (lane_b + pair);
+    constexpr int at = decltype(odd)::value * STAGE;
 #pragma unroll
-  for (int p = 0; p < STAGES - 1; ++p)
-    if (static_cast<uint32_t>(p) < steps) issue(p);
-  for (uint32_t s = 0; s < steps; ++s) {
-    // This thread's DMAs of step s are done when at most those of the later steps already issued
-    // (2 DMA per step) are in flight.
-    wait_vm(2 * DMA * min(steps - 1 - s, static_cast<uint32_t>(STAGES - 2)));
-    // A bare barrier: __syncthreads' fence would also wait for the later steps' loads. The empty
-    // asm statements keep the compiler from moving memory accesses across it; the waits above and
-    // the LDS reads of step s - 1, complete before its MFMAs, make it a full barrier for this ring.
+    for (int i = 0; i < 4; ++i) f.a[i] = *reinterpret_cast<const uint4_t*>(pa + at + 16 * i * KQ);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f.b[i] = *reinterpret_cast<const int4_t*>(pb + at + 16 * i * KQ);
+  };
+  auto multiply = [&](const Frags& f) {
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      // The row sums are taken by both wavefronts of a row (a branch would cut the step's
+      // instructions in pieces that cannot overlap); the left one's are used.
+      if constexpr (ROW_SUMS) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        raw[mt] = A_SIGNED ? static_cast<uint32_t>(__builtin_amdgcn_sdot4(static_cast<int>(f.a[mt][e]), 0x01010101,
+                                                                          static_cast<int>(raw[mt]), false))
+                           : __builtin_amdgcn_udot4(f.a[mt][e], 0x01010101u, raw[mt], false);
+      }
+      const int4_t af = __builtin_bit_cast(int4_t, f.a[mt] ^ aflip);
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f.b[nt], af, acc[mt][nt], 0, 0, 0);
+    }
+  };
+  // A bare barrier: __syncthreads' fence would also wait for the later stages' loads. The empty asm
+  // statements keep the compiler from moving memory accesses across it.
+  auto barrier = [&]() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (s + STAGES - 1 < steps) issue(s + STAGES - 1);
-    const uint8_t* sa = lds + (s % STAGES) * STAGE;
-    const uint8_t* sb = sa + kQT * KQ;
-#pragma unroll
-    for (int u = 0; u < SUB; ++u) {
-      const int c = kh * (PPR / KS) + 4 * u + g;  // this lane's 16-byte piece of the step's KQ bytes
-      int4_t af[4], bf[4];
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
-        const int row = 64 * wm + 16 * mt + r;
-        const uint4_t v = *reinterpret_cast<const uint4_t*>(sa + row * KQ + ((c ^ frag_swizzle<PPR>(row)) << 4));
-        if (wn == 0) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            raw[mt] = A_SIGNED ? static_cast<uint32_t>(__builtin_amdgcn_sdot4(static_cast<int>(v[e]), 0x01010101,
-                                                                              static_cast<int>(raw[mt]), false))
-                               : __builtin_amdgcn_udot4(v[e], 0x01010101u, raw[mt], false);
-        }
-        af[mt] = __builtin_bit_cast(int4_t, v ^ aflip);
-      }
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const int row = 64 * wn + 16 * nt + r;
-        bf[nt] = *reinterpret_cast<const int4_t*>(sb + row * KQ + ((c ^ frag_swizzle<PPR>(row)) << 4));
-      }
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
-          acc[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bf[nt], af[mt], acc[mt][nt], 0, 0, 0);
+  };
+  // Step s multiplies the fragments read in step s - 1 while those of step s + 1 come from LDS and
+  // stage s + 3 from memory. Ahead of its barrier a wavefront waits for its part of stage s + 1 and for
+  // its reads of step s; the barrier makes both everybody's: stage s + 1 is there, and stage
+  // (s - 1) % 4, which step s refills, was read whole before barrier s - 1. The steps at either end,
+  // which issue or read less, are written out: a branch around the reads would make the compiler wait
+  // for them ahead of the multiplications that they should overlap.
+  Frags fa, fb;
+  auto step = [&](uint32_t s, auto next_odd, const Frags& cur, Frags& next, auto in_flight, auto more) {
+    wait_vm<decltype(in_flight)::value>();
+    barrier();
+    // (Held in this order: left alone the compiler multiplies ahead of the barrier and reads last.)
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (decltype(more)::value) issue(s + 3);
+    read(s + 1, next_odd, next);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(cur);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr std::integral_constant<int, 2 * DMA> one{};  // one later stage's DMAs in flight
+  constexpr std::integral_constant<int, 0> none{};
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
+  issue(0);
+  issue(1);
+  if (steps > 2) {  // (steps is even: rows of k are padded to two of them)
+    issue(2);
+    wait_vm<4 * DMA>();
+    barrier();
+    read(0, even, fa);
+    for (uint32_t s = 0; s + 4 < steps; s += 2) {
+      step(s, odd, fa, fb, one, std::true_type{});
+      step(s + 1, even, fb, fa, one, std::true_type{});
     }
+    step(steps - 4, odd, fa, fb, one, std::true_type{});
+    step(steps - 3, even, fb, fa, one, std::false_type{});
+  } else {
+    wait_vm<2 * DMA>();
+    barrier();
+    read(0, even, fa);
   }
+  step(steps - 2, odd, fa, fb, none, std::false_type{});
+  multiply(fb);
   __syncthreads();  // every stage read: the LDS takes the other k-parts' sums
   // The k-parts of a quadrant add in a tree through LDS slots of 64 KiB (parts KS/2.. into
   // 0.., then ...), and A's row sums per part go to rs_part[part][row].
   constexpr int SLOT = 4 * 16 * 64;  // int4 entries of one slot: 4 quadrants x 16 tiles x 64 lanes
   auto* part = reinterpret_cast<int4_t*>(lds);
   auto* rs_part = reinterpret_cast<uint32_t*>(lds + (KS / 2) * SLOT * 16);
-  if (wn == 0) {
+  if (ROW_SUMS && wn == 0) {
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
       uint32_t v = raw[mt];
@@ -305,8 +356,10 @@ __global__ __launch_bounds__(64 * NW) void k_mmi_bt(const uint8_t* __restrict__ 
     }
     const uint32_t ca = oa - az;
     uint32_t rs = 0u - oa * K;
+    if constexpr (ROW_SUMS) {
 #pragma unroll
-    for (int p = 0; p < KS; ++p) rs += rs_part[p * kQT + ml];
+      for (int p = 0; p < KS; ++p) rs += rs_part[p * kQT + ml];
+    }
     int32_t* yrow = y + (static_cast<int64_t>(blockIdx.z) * M + m) * N;
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
@@ -359,6 +412,7 @@ int tmh_int8_weight_prepare(tmh_ctx* ctx, const void* d_b, int b_dtype, const vo
   w->K = K;
   w->Kp = Kp;
   w->N = N;
+  w->symmetric = b_dtype == TMH_S8 && !d_b_zero;
   // The column terms are padded to whole 16-byte groups, which the GEMM loads whole.
   const size_t terms = static_cast<size_t>((N + 3) / 4 * 4) * 4;
   int st = check_hip(ctx, hipMalloc(reinterpret_cast<void**>(&w->d_bt), static_cast<size_t>(N * Kp)), "hipMalloc");
@@ -430,17 +484,18 @@ int tmh_matmul_integer_prepared(tmh_ctx* ctx, const void* d_a, int a_dtype, cons
   const dim3 grid(static_cast<unsigned>((w->N + kQT - 1) / kQT), static_cast<unsigned>((M + kQT - 1) / kQT),
                   static_cast<unsigned>(batch));
   const bool y_vec = w->N % 4 == 0 && reinterpret_cast<uintptr_t>(d_y) % 16 == 0;
-  // 256-byte k-steps in two stages, eight wavefronts: 20.5 us at 2048^3 u8 x u8 (840 TOP/s)
-  // against 21.0 us for 128-byte steps in three stages, 22.0 in four, and 20.7 with sixteen
-  // wavefronts; the unprepared kernel takes 28.5 us.
-  constexpr int kLds = 2 * 2 * kQT * 256;
-  auto* kernel = a_dtype == TMH_S8 ? k_mmi_bt<true, 256, 2> : k_mmi_bt<false, 256, 2>;
-  static const hipError_t attr[2] = {
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mmi_bt<true, 256, 2>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mmi_bt<false, 256, 2>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds)};
+  constexpr int kLds = 4 * 2 * kQT * 128;
+  // A symmetric B has no use for A's row sums (each is multiplied by ob - bz_n = 0).
+  using Kernel = decltype(&k_mmi_bt<true, true, 128, 4>);
+  static const Kernel kernels[4] = {&k_mmi_bt<false, true, 128, 4>, &k_mmi_bt<true, true, 128, 4>,
+                                    &k_mmi_bt<false, false, 128, 4>, &k_mmi_bt<true, false, 128, 4>};
+  static const hipError_t attr[4] = {
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kernels[0]), hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kernels[1]), hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kernels[2]), hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kernels[3]), hipFuncAttributeMaxDynamicSharedMemorySize, kLds)};
   (void)attr;
+  const Kernel kernel = kernels[(a_dtype == TMH_S8 ? 1 : 0) + (w->symmetric ? 2 : 0)];
   kernel<<<grid, 512, kLds, s>>>(static_cast<const uint8_t*>(d_a), w->d_bt, w->d_cs, w->d_cb,
                                  static_cast<const uint8_t*>(d_a_zero), a_zero_count, static_cast<uint32_t>(M),
                                  static_cast<uint32_t>(w->K), static_cast<uint32_t>(w->Kp), static_cast<uint32_t>(w->N),
