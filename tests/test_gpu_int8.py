@@ -229,6 +229,17 @@ def test_matmul_integer_prepared_matches_oracle(ctx, case):
     _check_prepared(ctx, case)
 
 
+# The prepared GEMM's ring of 128-byte steps (two, four, six and eight of them, whole and ending in
+# padding), with and without A's row sums (an s8 B without zero points has no use for them).
+@pytest.mark.parametrize("k", [16, 256, 272, 496, 512, 528, 768, 1024, 1040])
+@pytest.mark.parametrize("a_type", ["u8", "s8"])
+@pytest.mark.parametrize("b_type,b_zero", [("s8", None), ("s8", "col"), ("u8", None)])
+def test_matmul_integer_prepared_steps(ctx, k, a_type, b_type, b_zero):
+    case = (1, 135, k, 140, a_type, b_type, "row", b_zero)
+    print(f"matmul_integer prepared {case}", flush=True)
+    _check_prepared(ctx, case)
+
+
 def _draw_prepared(seed):
     """A seeded random MatMulInteger over a prepared B: K a multiple of 16 (what preparation
     takes), M and N ragged against the 128-row tiles, batches, every signedness and zero-point
