@@ -32,6 +32,10 @@ using namespace tmh;
 namespace {
 
 constexpr int kMoeRows = 32;  // rows per work item of the general product
+// Chunks of weights and of A on their way while one is multiplied: two, but one for swiglu over 64
+// rows, whose register sets for a third chunk leave one workgroup to a CU (512 tokens of 128 experts
+// 120.6 us against 115).
+constexpr int moe_ahead(int epi, int mt) { return epi == 2 && mt == 4 ? 1 : 2; }
 // Tokens up to which one workgroup routes and plans (k_moe_route_plan): two for each of its wavefronts.
 constexpr int kFusedRouteTokens = 32;
 
@@ -327,8 +331,8 @@ enum : int { EPI_STORE = 0, EPI_ACT = 1, EPI_GLU = 2 };
 // one work item, f16 in and out with f32 sums (v_mfma_f32_16x16x32_f16). src(row) = perm[row] /
 // perm_div when perm is given (rows gathered from the tokens), else row. Each of the eight
 // wavefronts owns one 16-column output tile (and, for EPI_GLU, the matching tile of the second
-// weight) over all of K; the item's A rows pass through LDS one chunk at a time, double
-// buffered, with the next chunk's weights in flight.
+// weight) over all of K; the item's A rows pass through LDS one chunk at a time, with the next two
+// chunks' weights and rows in flight.
 // (The body; k_moe_gemm_f16 and its stamping build k_moe_gemm_f16_tl below are the kernels.)
 template <int BITS, bool HAS_ZP, bool SPLIT, int EPI, int MT, bool TL>
 __device__ __forceinline__ void moe_gemm_f16(
@@ -348,9 +352,12 @@ __device__ __forceinline__ void moe_gemm_f16(
   constexpr int PPR = CW / 8;                    // 16-byte pieces per row
   constexpr int ROWS = 16 * MT;                  // rows per work item
   constexpr int PIECES = ROWS * PPR;             // per chunk
-  constexpr int LOADS = (PIECES + 511) / 512;    // per thread
+  constexpr int DMA = (PIECES + 511) / 512;      // load instructions of a wavefront per chunk of A
   constexpr int NW = EPI == EPI_GLU ? 2 : 1;
-  __shared__ __align__(16) uint8_t lds[2 * ROWS * ROWB];
+  constexpr int STEP_LOADS = DMA + NW * (1 + NJ * (HAS_ZP ? 2 : 1));  // of a wavefront per step
+  constexpr int AHEAD = moe_ahead(EPI, MT);
+  constexpr uint32_t STAGES = AHEAD + 1;
+  extern __shared__ __align__(16) uint8_t lds[];  // STAGES chunks of the item's rows of A
   if (static_cast<int>(blockIdx.y) >= *n_items) {
     if constexpr (TL) tl_stamp(tl, tl0);
     return;
@@ -377,40 +384,39 @@ __device__ __forceinline__ void moe_gemm_f16(
     z_rsrc[v] = buffer_rsrc(v ? zp2 : zp, HAS_ZP ? zp_byte<BITS>(n_params) : 0u);
     tile0[v] = static_cast<uint32_t>(it.e * tiles_per_expert + lt_of(0) + (v ? tile_off2 : 0));
   }
-  // A pieces this thread brings to LDS: row p / PPR, piece p % PPR of p = (tid + 512 l) mod
-  // PIECES (rows past the item, and k past K, read zeros). Where 512 * LOADS exceeds PIECES, two
-  // threads store the same piece, the same bytes.
-  uint32_t a_src[LOADS];
-  int a_dst[LOADS], a_k[LOADS];
+  // A goes global -> LDS by buffer_load ... lds: instruction j of this wavefront fills 64 slots from
+  // p = ((wave DMA + j) 64) mod PIECES on, each lane loading the piece that belongs in its slot of
+  // the swizzled rows (rows past the item, and k past K, read zeros; where 512 DMA exceeds PIECES two
+  // wavefronts bring the same bytes).
+  uint32_t a_src[DMA];
+  int a_k[DMA];
 #pragma unroll
-  for (int l = 0; l < LOADS; ++l) {
-    const int p = (tid + 512 * l) % PIECES;
-    const int row = p / PPR, piece = p % PPR;
+  for (int j = 0; j < DMA; ++j) {
+    const int p = ((wave * DMA + j) * 64) % PIECES + lane;
+    const int row = p / PPR, piece = a_slot_moe<BITS>(row, p % PPR);  // the swizzle is its own inverse
     const int src = row < it.rows ? (perm ? perm[it.row0 + row] / perm_div : it.row0 + row) : -1;
-    a_src[l] = src >= 0 ? static_cast<uint32_t>(src) * lda * 2 + piece * 16 : 0x80000000u;
-    a_dst[l] = row * ROWB + a_slot_moe<BITS>(row, piece) * 16;
-    a_k[l] = piece * 8;
+    a_src[j] = src >= 0 ? static_cast<uint32_t>(src) * lda * 2 + piece * 16 : 0x80000000u;
+    a_k[j] = piece * 8;
   }
-  auto load_a = [&](uint32_t c, uint4_t (&v)[LOADS]) {
+  auto load_a = [&](uint32_t c, uint32_t stage, bool real) {
 #pragma unroll
-    for (int l = 0; l < LOADS; ++l) {
-      const bool in_k = static_cast<int>(c) * CW + a_k[l] < lda;  // lda = K, a multiple of 8
-      v[l] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, in_k ? a_src[l] + c * CW * 2 : 0x80000000u, 0, 0);
+    for (int j = 0; j < DMA; ++j) {
+      const bool in_k = real && static_cast<int>(c) * CW + a_k[j] < lda;  // lda = K, a multiple of 8
+      lds_dma16(a_rsrc, lds + stage * (ROWS * ROWB) + (((wave * DMA + j) * 64) % PIECES) * 16,
+                in_k ? a_src[j] + c * CW * 2 : 0x80000000u, 0);
     }
-  };
-  auto store_a = [&](int buf, const uint4_t (&v)[LOADS]) {
-#pragma unroll
-    for (int l = 0; l < LOADS; ++l) *reinterpret_cast<uint4_t*>(lds + buf * ROWS * ROWB + a_dst[l]) = v[l];
   };
   struct WStage {
     uint4_t w[NW];
     uint32_t s[NW][NJ], z[NW][NJ];
   };
-  auto load_w = [&](int gi, uint32_t c, WStage& st) {
+  // (A wavefront without a tile in the last group reads the one before and stores nothing; a step past
+  // the last, real = false, reads zeros: the loads of every step are the same in number.)
+  auto load_w = [&](int gi, uint32_t c, bool real, WStage& st) {
 #pragma unroll
     for (int v = 0; v < NW; ++v) {
-      const uint32_t tile = tile0[v] + 8u * static_cast<uint32_t>(gi);
-      st.w[v] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc[v], (tile * nch * 64 + lane) * 16, c * 1024, 0);
+      const uint32_t tile = tile0[v] + 8u * static_cast<uint32_t>(active_g(gi) ? gi : 0);
+      st.w[v] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc[v], real ? (tile * nch * 64 + lane) * 16 : 0x80000000u, c * 1024, 0);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
         const uint32_t e = ((tile * nch + c) * nbc + ((g * GW + 8 * j * (SPLIT ? 1 : 0)) >> bsc_shift)) * 16 + r;
@@ -455,60 +461,80 @@ __device__ __forceinline__ void moe_gemm_f16(
   // The chunk loop over the workgroup's groups (steps s: group s / nch, chunk s % nch),
   // specialized for the m-tiles that hold rows of this item (MA of MT, uniform per workgroup): an
   // item of 17-32 rows runs half the MFMAs and LDS reads of a full one.
+  // Step s multiplies chunk s while the weights and rows of the next AHEAD chunks are on their way:
+  // ahead of its barrier a wavefront waits for its own loads of step s alone (a bare barrier:
+  // __syncthreads would wait for the later ones too, a memory latency per chunk), the barrier makes
+  // the rows everybody's and frees the stage of step s - 1, read whole by then, for step s + AHEAD.
   auto run = [&](auto ma) {
     constexpr int MA = decltype(ma)::value;
-    uint4_t av[LOADS];
-    WStage cur, next;
-    load_a(0, av);
-    if (active_g(0)) load_w(0, 0, cur);
-    store_a(0, av);
-    __syncthreads();
+    WStage w0, w1, w2;
     const uint32_t total = static_cast<uint32_t>(ng) * nch;
-    uint32_t c = 0;
-    int gi = 0;
-    for (uint32_t s = 0; s < total; ++s) {
-      const bool more = s + 1 < total;
-      const bool last_chunk = c + 1 == nch;
-      const uint32_t c1 = last_chunk ? 0u : c + 1;
-      const int gi1 = last_chunk ? gi + 1 : gi;
-      if (more) {
-        load_a(c1, av);
-        if (active_g(gi1)) load_w(gi1, c1, next);
+    uint32_t cl = 0, sl = 0, stage_l = 0;  // chunk, step and stage of the next loads
+    int gl = 0;
+    auto load_next = [&](WStage& st) {
+      load_a(cl, stage_l, sl < total);
+      load_w(gl, cl, sl < total, st);
+      ++sl;
+      stage_l = stage_l + 1 == STAGES ? 0 : stage_l + 1;
+      if (++cl == nch) {
+        cl = 0;
+        ++gl;
       }
-      if (active_g(gi)) {
-        const uint8_t* abase = lds + (s & 1) * ROWS * ROWB;
+    };
+    uint32_t c = 0, stage = 0;
+    int gi = 0;
+    auto step = [&](const WStage& cur, WStage& far) {
+      constexpr int kWait = (AHEAD - 1) * STEP_LOADS;  // the loads of step s + 1 may stay in flight
+      __builtin_amdgcn_s_waitcnt((kWait & 15) | (7 << 4) | ((kWait >> 4) << 14));
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      load_next(far);
+      __builtin_amdgcn_sched_barrier(0);
+      const uint8_t* abase = lds + stage * (ROWS * ROWB);
 #pragma unroll
-        for (int i = 0; i < STEPS; ++i) {
-          const int piece = g * (GW / 8) + i;
-          half8_t af[MA];
+      for (int i = 0; i < STEPS; ++i) {
+        const int piece = g * (GW / 8) + i;
+        half8_t af[MA];
+#pragma unroll
+        for (int mt = 0; mt < MA; ++mt)
+          af[mt] = *reinterpret_cast<const half8_t*>(abase + (mt * 16 + r) * ROWB + a_slot_moe<BITS>(mt * 16 + r, piece) * 16);
+        const int j = SPLIT ? i : 0;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) {
+          const uint32_t zq = HAS_ZP ? 0x6400u + zp_field<BITS>(cur.z[v][j], zp_shift<BITS>(r)) : 0x6400u + (1u << (BITS - 1));
+          const half8_t b = unpack_step<BITS>(cur.w[v], i, __builtin_bit_cast(half2_t, zq | (zq << 16)),
+                                              __builtin_bit_cast(half2_t, cur.s[v][j] | (cur.s[v][j] << 16)));
 #pragma unroll
           for (int mt = 0; mt < MA; ++mt)
-            af[mt] = *reinterpret_cast<const half8_t*>(abase + (mt * 16 + r) * ROWB + a_slot_moe<BITS>(mt * 16 + r, piece) * 16);
-          const int j = SPLIT ? i : 0;
-#pragma unroll
-          for (int v = 0; v < NW; ++v) {
-            const uint32_t zq = HAS_ZP ? 0x6400u + zp_field<BITS>(cur.z[v][j], zp_shift<BITS>(r)) : 0x6400u + (1u << (BITS - 1));
-            const half8_t b = unpack_step<BITS>(cur.w[v], i, __builtin_bit_cast(half2_t, zq | (zq << 16)),
-                                                __builtin_bit_cast(half2_t, cur.s[v][j] | (cur.s[v][j] << 16)));
-#pragma unroll
-            for (int mt = 0; mt < MA; ++mt)
-              acc[v][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, af[mt], acc[v][mt], 0, 0, 0);
-          }
-        }
-        if (last_chunk) {
-          store_group(gi);
-#pragma unroll
-          for (int v = 0; v < NW; ++v)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) acc[v][mt] = float4_t{0.f, 0.f, 0.f, 0.f};
+            acc[v][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, af[mt], acc[v][mt], 0, 0, 0);
         }
       }
-      if (more) store_a((s + 1) & 1, av);
-      __syncthreads();
-      if (more) cur = next;
-      c = c1;
-      gi = gi1;
+      stage = stage + 1 == STAGES ? 0 : stage + 1;
+      if (++c == nch) {
+        if (active_g(gi)) store_group(gi);
+#pragma unroll
+        for (int v = 0; v < NW; ++v)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) acc[v][mt] = float4_t{0.f, 0.f, 0.f, 0.f};
+        c = 0;
+        ++gi;
+      }
+    };
+    load_next(w0);
+    if constexpr (AHEAD == 2) load_next(w1);
+    for (uint32_t s = 0;;) {
+      step(w0, AHEAD == 2 ? w2 : w1);
+      if (++s == total) break;
+      step(w1, w0);
+      if (++s == total) break;
+      if constexpr (AHEAD == 2) {
+        step(w2, w1);
+        if (++s == total) break;
+      }
     }
+    __builtin_amdgcn_s_waitcnt(0);  // the loads past the last step write the LDS: done before it is given back
   };
   const int used = (it.rows + 15) / 16;
   if (MT >= 4 && used > 2) {
@@ -978,10 +1004,17 @@ void launch_moe_f16_e(const tmh_weight* w, int tpe, const void* A, int a_rows, i
       static_cast<const _Float16*>(A), a_rows, lda, perm, perm_div, items, n_items, ep.bias1,        \
       ep.bias2, ep.bias_dt, ep.bias_ld, ep.act, ep.alpha, ep.beta, ep.limit, static_cast<_Float16*>(out), ldo,       \
       ep.out_perm
+  constexpr int kLds = (moe_ahead(EPI, MT) + 1) * 16 * MT * (512 / BITS) * 2;
+  static const hipError_t attr[2] = {
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_moe_gemm_f16<BITS, HAS_ZP, SPLIT, EPI, MT>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_moe_gemm_f16_tl<BITS, HAS_ZP, SPLIT, EPI, MT>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds)};
+  (void)attr;
   if (uint32_t* tl = timeline_slots(TMH_TL_MOE_GEMM, static_cast<int64_t>(grid.x) * grid.y * 8))
-    k_moe_gemm_f16_tl<BITS, HAS_ZP, SPLIT, EPI, MT><<<grid, 512, 0, s>>>(TMH_MOE_ARGS, tl);
+    k_moe_gemm_f16_tl<BITS, HAS_ZP, SPLIT, EPI, MT><<<grid, 512, kLds, s>>>(TMH_MOE_ARGS, tl);
   else
-    k_moe_gemm_f16<BITS, HAS_ZP, SPLIT, EPI, MT><<<grid, 512, 0, s>>>(TMH_MOE_ARGS);
+    k_moe_gemm_f16<BITS, HAS_ZP, SPLIT, EPI, MT><<<grid, 512, kLds, s>>>(TMH_MOE_ARGS);
 #undef TMH_MOE_ARGS
 }
 
