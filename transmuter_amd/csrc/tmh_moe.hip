@@ -484,7 +484,10 @@ __device__ __forceinline__ void moe_gemm_f16(
     uint32_t c = 0, stage = 0;
     int gi = 0;
     auto step = [&](const WStage& cur, WStage& far) {
-      constexpr int kWait = (AHEAD - 1) * STEP_LOADS;  // the loads of step s + 1 may stay in flight
+      // The loads of step s + 1 may stay in flight. (The count holds as long as none of them is moved past
+      // the barrier, which the compiler may do with the weights' ones: over all paths of every build's
+      // assembly no row load older than step s + 1 is in flight at a barrier. Look again when this changes.)
+      constexpr int kWait = (AHEAD - 1) * STEP_LOADS;
       __builtin_amdgcn_s_waitcnt((kWait & 15) | (7 << 4) | ((kWait >> 4) << 14));
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
