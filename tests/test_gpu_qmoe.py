@@ -207,12 +207,13 @@ def test_qmoe_routing_ties_among_many_experts(ctx, e):
     assert np.abs(got - ref).max() <= 1e-2 * scale, f"max difference {np.abs(got - ref).max()} (max |ref| {scale})"
 
 
-def test_qmoe_fc3_without_zero_points_beside_fc1_with_them(ctx):
+@pytest.mark.parametrize("t", [20, 130], ids=["t20", "t130_items_of_64"])
+def test_qmoe_fc3_without_zero_points_beside_fc1_with_them(ctx, t):
     """fc1 with packed zero points and fc3 without (each QMoE input has its own, moe.ex:45): the
     swiglu product must read each weight with its own layout."""
-    print("qmoe fc1 zp, fc3 none", flush=True)
+    print(f"qmoe fc1 zp, fc3 none, t={t}", flush=True)
     rng = np.random.default_rng(9)
-    e, k, t, h, n1 = 8, 2, 20, 64, 32
+    e, k, h, n1 = 8, 2, 64, 32
     w1, s1, z1 = _weights(rng, e, n1, h, 4, 32, True, "f16")
     w3, s3, _ = _weights(rng, e, n1, h, 4, 32, False, "f16")
     w2, s2, z2 = _weights(rng, e, h, n1, 4, 32, True, "f16")
@@ -278,4 +279,24 @@ FEW_CASES = [
 @pytest.mark.parametrize("skew", [0.0, 6.0])
 def test_qmoe_few_rows(ctx, case, skew):
     print(f"qmoe few rows {case} skew={skew}", flush=True)
+    _check_qmoe(ctx, case, skew)
+
+
+# fc1 that is not fused with its activation (interleaved swiglu; halves off 16 columns): its own product
+# and k_moe_activate, with items of 64 rows (over 24 rows an expert), 32 and 16 (few rows), experts
+# with more than 32 rows among them.
+UNFUSED_CASES = [
+    ("f16", 4, 2, 90, 64, 96, "swiglu", 1, False, 4, 32, True, True, 7.0),
+    ("f16", 32, 4, 512, 128, 64, "swiglu", 1, False, 4, 32, False, False, 0.0),
+    ("f16", 6, 3, 100, 80, 48, "swiglu", 2, False, 8, 16, True, True, 0.0),
+    ("f16", 8, 2, 70, 144, 176, "swiglu", 1, False, 4, 64, True, False, 0.0),
+    ("f16", 8, 2, 12, 144, 80, "swiglu", 1, False, 4, 32, True, True, 7.0),
+    ("f16", 8, 2, 12, 144, 80, "swiglu", 2, False, 8, 32, False, False, 0.0),
+]
+
+
+@pytest.mark.parametrize("case", UNFUSED_CASES, ids=lambda c: "{}_E{}_k{}_T{}_H{}_N{}_{}{}_b{}_bs{}".format(*c[:8], c[9], c[10]))
+@pytest.mark.parametrize("skew", [0.0, 6.0])
+def test_qmoe_unfused_fc1(ctx, case, skew):
+    print(f"qmoe unfused fc1 {case} skew={skew}", flush=True)
     _check_qmoe(ctx, case, skew)

@@ -974,6 +974,15 @@ int bsc_shift_moe(const tmh_weight* w) {
   return s;
 }
 
+// The work items of a call (the plan's), their number on the device and at most, and the rows of each:
+// every product of the call takes the build that covers them (k_moe_rows 16, the others 32 or 64).
+struct MoeWork {
+  const int4* items;
+  const int* n_items;
+  int max_items, rows;
+  bool few;  // k_moe_rows
+};
+
 // The epilogue of a fast grouped product.
 struct MoeEpilogue {
   int kind = EPI_STORE;
@@ -983,14 +992,12 @@ struct MoeEpilogue {
   const void *bias1 = nullptr, *bias2 = nullptr;
   int bias_dt = TMH_F32, bias_ld = 0, act = ACT_IDENTITY;
   float alpha = 1.f, beta = 0.f, limit = 0.f;
-  int rows = 32;                   // rows per work item: 32 or 64 (k_moe_rows: 16)
-  bool few_rows = false;           // the product for items of few rows, k_moe_rows
   const int* out_perm = nullptr;   // output row of each sorted row (else the sorted row itself)
 };
 
 template <int BITS, bool HAS_ZP, bool SPLIT, int EPI, int MT>
 void launch_moe_f16_e(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
-                      const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
+                      const MoeWork& work, void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
   const tmh_weight* w2 = ep.w2 ? ep.w2 : w;
   // Groups of eight output tiles per workgroup, one after the other: the stored products (fc2,
   // many groups per item) run four, so the workgroups' prologues and the last partial round of
@@ -998,13 +1005,13 @@ void launch_moe_f16_e(const tmh_weight* w, int tpe, const void* A, int a_rows, i
   const int groups = (ep.out_tiles + 7) / 8;
   const char* gpw_env = std::getenv("TMH_MOE_GPW");
   const int gpw = gpw_env ? std::max(1, std::atoi(gpw_env)) : (EPI == EPI_STORE && groups >= 16 ? 4 : 1);
-  const dim3 grid(static_cast<unsigned>((groups + gpw - 1) / gpw), static_cast<unsigned>(max_items));
+  const dim3 grid(static_cast<unsigned>((groups + gpw - 1) / gpw), static_cast<unsigned>(work.max_items));
 #define TMH_MOE_ARGS                                                                                                   \
   reinterpret_cast<const uint4_t*>(w->d_q), static_cast<const uint16_t*>(w->d_scale),                                 \
       static_cast<const uint8_t*>(w->d_zero), reinterpret_cast<const uint4_t*>(w2->d_q),                              \
       static_cast<const uint16_t*>(w2->d_scale), static_cast<const uint8_t*>(w2->d_zero), ep.tile_off2,               \
       static_cast<int>(w->ntiles), static_cast<int>(w->nchunks), w->nbc, bsc_shift_moe(w), tpe, ep.out_tiles, gpw,    \
-      static_cast<const _Float16*>(A), a_rows, lda, perm, perm_div, items, n_items, ep.bias1,        \
+      static_cast<const _Float16*>(A), a_rows, lda, perm, perm_div, work.items, work.n_items, ep.bias1,        \
       ep.bias2, ep.bias_dt, ep.bias_ld, ep.act, ep.alpha, ep.beta, ep.limit, static_cast<_Float16*>(out), ldo,       \
       ep.out_perm
   constexpr int kLds = (moe_ahead(EPI, MT) + 1) * 16 * MT * (512 / BITS) * 2;
@@ -1023,40 +1030,40 @@ void launch_moe_f16_e(const tmh_weight* w, int tpe, const void* A, int a_rows, i
 
 template <int BITS, bool HAS_ZP, bool SPLIT, int EPI, int TN, int NW>
 void go_moe_rows(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
-                 const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep,
+                 const MoeWork& work, void* out, int ldo, const MoeEpilogue& ep,
                  hipStream_t s) {
   const tmh_weight* w2 = ep.w2 ? ep.w2 : w;
-  const dim3 grid(static_cast<unsigned>((ep.out_tiles + TN - 1) / TN), static_cast<unsigned>(max_items));
+  const dim3 grid(static_cast<unsigned>((ep.out_tiles + TN - 1) / TN), static_cast<unsigned>(work.max_items));
   k_moe_rows<BITS, HAS_ZP, SPLIT, EPI, TN, NW><<<grid, 64 * NW, 0, s>>>(
       reinterpret_cast<const uint4_t*>(w->d_q), static_cast<const uint16_t*>(w->d_scale),
       static_cast<const uint8_t*>(w->d_zero), reinterpret_cast<const uint4_t*>(w2->d_q),
       static_cast<const uint16_t*>(w2->d_scale), static_cast<const uint8_t*>(w2->d_zero), ep.tile_off2,
       static_cast<int>(w->ntiles), static_cast<int>(w->nchunks), w->nbc, bsc_shift_moe(w), tpe, ep.out_tiles,
-      static_cast<const _Float16*>(A), a_rows, lda, perm, perm_div, items, n_items, ep.bias1, ep.bias2, ep.bias_dt,
+      static_cast<const _Float16*>(A), a_rows, lda, perm, perm_div, work.items, work.n_items, ep.bias1, ep.bias2, ep.bias_dt,
       ep.bias_ld, ep.act, ep.alpha, ep.beta, ep.limit, static_cast<_Float16*>(out), ldo, ep.out_perm);
 }
 
 template <int BITS, bool HAS_ZP, bool SPLIT, int EPI>
 void launch_moe_rows_e(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
-                       const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep,
+                       const MoeWork& work, void* out, int ldo, const MoeEpilogue& ep,
                        hipStream_t s) {
   // One output tile (of both weights) over four wavefronts for swiglu; else two tiles, over two
   // wavefronts where K is short (8 tokens of 128 experts, fc1 and fc3 with 16 chunks: 1,4 47.7 us a
   // call, 1,2 47.9, 1,8 52.3, 2,4 50.2; fc2 with 6: 2,2 47.6, 1,2 48.1, 2,4 49.1, 4,2 50.5).
   if constexpr (EPI == EPI_GLU)
-    go_moe_rows<BITS, HAS_ZP, SPLIT, EPI, 1, 4>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s);
+    go_moe_rows<BITS, HAS_ZP, SPLIT, EPI, 1, 4>(w, tpe, A, a_rows, lda, perm, perm_div, work, out, ldo, ep, s);
   else if (w->nchunks <= 8)
-    go_moe_rows<BITS, HAS_ZP, SPLIT, EPI, 2, 2>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s);
+    go_moe_rows<BITS, HAS_ZP, SPLIT, EPI, 2, 2>(w, tpe, A, a_rows, lda, perm, perm_div, work, out, ldo, ep, s);
   else
-    go_moe_rows<BITS, HAS_ZP, SPLIT, EPI, 2, 4>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s);
+    go_moe_rows<BITS, HAS_ZP, SPLIT, EPI, 2, 4>(w, tpe, A, a_rows, lda, perm, perm_div, work, out, ldo, ep, s);
 }
 
 template <int BITS, bool HAS_ZP, bool SPLIT>
 void launch_moe_rows(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
-                     const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep,
+                     const MoeWork& work, void* out, int ldo, const MoeEpilogue& ep,
                      hipStream_t s) {
 #define TMH_MOE_ROWS(E) \
-  launch_moe_rows_e<BITS, HAS_ZP, SPLIT, E>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s)
+  launch_moe_rows_e<BITS, HAS_ZP, SPLIT, E>(w, tpe, A, a_rows, lda, perm, perm_div, work, out, ldo, ep, s)
   if (ep.kind == EPI_GLU) TMH_MOE_ROWS(EPI_GLU);
   else if (ep.kind == EPI_ACT) TMH_MOE_ROWS(EPI_ACT);
   else TMH_MOE_ROWS(EPI_STORE);
@@ -1065,10 +1072,10 @@ void launch_moe_rows(const tmh_weight* w, int tpe, const void* A, int a_rows, in
 
 template <int BITS, bool HAS_ZP, bool SPLIT>
 void launch_moe_f16_v(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
-                      const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
+                      const MoeWork& work, void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
 #define TMH_MOE_EPI(E, MT) \
-  launch_moe_f16_e<BITS, HAS_ZP, SPLIT, E, MT>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s)
-  if (ep.rows == 64) {
+  launch_moe_f16_e<BITS, HAS_ZP, SPLIT, E, MT>(w, tpe, A, a_rows, lda, perm, perm_div, work, out, ldo, ep, s)
+  if (work.rows == 64) {
     if (ep.kind == EPI_GLU) TMH_MOE_EPI(EPI_GLU, 4);
     else if (ep.kind == EPI_ACT) TMH_MOE_EPI(EPI_ACT, 4);
     else TMH_MOE_EPI(EPI_STORE, 4);
@@ -1082,12 +1089,12 @@ void launch_moe_f16_v(const tmh_weight* w, int tpe, const void* A, int a_rows, i
 
 template <int BITS>
 void launch_moe_f16(const tmh_weight* w, int tpe, const void* A, int a_rows, int lda, const int* perm, int perm_div,
-                    const int4* items, const int* n_items, int max_items, void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
+                    const MoeWork& work, void* out, int ldo, const MoeEpilogue& ep, hipStream_t s) {
   const bool zp = w->zp_kind == TMH_ZP_PACKED;
   const bool split = w->block_size < (512 / BITS) / 4;
   if constexpr (BITS != 2) {
-    if (ep.few_rows) {
-#define TMH_MOE_FEW(Z, S) launch_moe_rows<BITS, Z, S>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s)
+    if (work.few) {
+#define TMH_MOE_FEW(Z, S) launch_moe_rows<BITS, Z, S>(w, tpe, A, a_rows, lda, perm, perm_div, work, out, ldo, ep, s)
       if (zp && split) TMH_MOE_FEW(true, true);
       else if (zp) TMH_MOE_FEW(true, false);
       else if (split) TMH_MOE_FEW(false, true);
@@ -1097,7 +1104,7 @@ void launch_moe_f16(const tmh_weight* w, int tpe, const void* A, int a_rows, int
     }
   }
 #define TMH_MOE_F16(Z, S) \
-  launch_moe_f16_v<BITS, Z, S>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s)
+  launch_moe_f16_v<BITS, Z, S>(w, tpe, A, a_rows, lda, perm, perm_div, work, out, ldo, ep, s)
   if (zp && split) TMH_MOE_F16(true, true);
   else if (zp) TMH_MOE_F16(true, false);
   else if (split) TMH_MOE_F16(false, true);
@@ -1107,32 +1114,32 @@ void launch_moe_f16(const tmh_weight* w, int tpe, const void* A, int a_rows, int
 
 template <int BITS, int WDT>
 void launch_moe_general_w(const tmh_weight* w, int tpe, const void* A, int a_dt, int lda, const int* perm, int perm_div,
-                          const int4* items, const int* n_items, int max_items, void* out, int out_dt, int ldo, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(tpe), static_cast<unsigned>(max_items));
+                          const MoeWork& work, void* out, int out_dt, int ldo, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(tpe), static_cast<unsigned>(work.max_items));
   const auto* qt = reinterpret_cast<const uint4_t*>(w->d_q);
   const int sh = bsc_shift_moe(w);
   if (w->zp_kind == TMH_ZP_PACKED)
     k_moe_gemm_general<BITS, WDT, TMH_ZP_PACKED><<<grid, 256, 0, s>>>(
         qt, w->d_scale, w->d_zero, static_cast<int>(w->nchunks), w->nbc, sh, tpe, static_cast<int>(w->K), A, a_dt, lda,
-        perm, perm_div, items, n_items, out, out_dt, ldo);
+        perm, perm_div, work.items, work.n_items, out, out_dt, ldo);
   else
     k_moe_gemm_general<BITS, WDT, TMH_ZP_NONE><<<grid, 256, 0, s>>>(
         qt, w->d_scale, w->d_zero, static_cast<int>(w->nchunks), w->nbc, sh, tpe, static_cast<int>(w->K), A, a_dt, lda,
-        perm, perm_div, items, n_items, out, out_dt, ldo);
+        perm, perm_div, work.items, work.n_items, out, out_dt, ldo);
 }
 
 template <int BITS>
 void launch_moe_general(const tmh_weight* w, int tpe, const void* A, int a_dt, int lda, const int* perm, int perm_div,
-                        const int4* items, const int* n_items, int max_items, void* out, int out_dt, int ldo, hipStream_t s) {
+                        const MoeWork& work, void* out, int out_dt, int ldo, hipStream_t s) {
   switch (w->wdtype) {
     case TMH_F16:
-      launch_moe_general_w<BITS, DT_F16>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, out_dt, ldo, s);
+      launch_moe_general_w<BITS, DT_F16>(w, tpe, A, a_dt, lda, perm, perm_div, work, out, out_dt, ldo, s);
       break;
     case TMH_BF16:
-      launch_moe_general_w<BITS, DT_BF16>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, out_dt, ldo, s);
+      launch_moe_general_w<BITS, DT_BF16>(w, tpe, A, a_dt, lda, perm, perm_div, work, out, out_dt, ldo, s);
       break;
     default:
-      launch_moe_general_w<BITS, DT_F32>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, out_dt, ldo, s);
+      launch_moe_general_w<BITS, DT_F32>(w, tpe, A, a_dt, lda, perm, perm_div, work, out, out_dt, ldo, s);
   }
 }
 
@@ -1147,21 +1154,22 @@ bool moe_fast(const tmh_weight* w, int a_dt, const void* A, int a_rows, int lda)
 // One grouped product: rows (gathered through perm when given) times each row's expert. The
 // fast path applies the epilogue; the general path stores the sums (EPI_STORE only).
 void moe_gemm(const tmh_weight* w, int experts, const void* A, int a_dt, int a_rows, int lda, const int* perm,
-              int perm_div, const int4* items, const int* n_items, int max_items, void* out, int ldo, hipStream_t s, MoeEpilogue ep = MoeEpilogue()) {
+              int perm_div, const MoeWork& work, void* out, int ldo, hipStream_t s,
+              MoeEpilogue ep = MoeEpilogue()) {
   const int tpe = static_cast<int>(w->N / experts / 16);
   if (moe_fast(w, a_dt, A, a_rows, lda)) {
     if (ep.out_tiles == 0) ep.out_tiles = tpe;
     switch (w->bits) {
-      case 2: launch_moe_f16<2>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s); break;
-      case 4: launch_moe_f16<4>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s); break;
-      default: launch_moe_f16<8>(w, tpe, A, a_rows, lda, perm, perm_div, items, n_items, max_items, out, ldo, ep, s);
+      case 2: launch_moe_f16<2>(w, tpe, A, a_rows, lda, perm, perm_div, work, out, ldo, ep, s); break;
+      case 4: launch_moe_f16<4>(w, tpe, A, a_rows, lda, perm, perm_div, work, out, ldo, ep, s); break;
+      default: launch_moe_f16<8>(w, tpe, A, a_rows, lda, perm, perm_div, work, out, ldo, ep, s);
     }
     return;
   }
   switch (w->bits) {
-    case 2: launch_moe_general<2>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, a_dt, ldo, s); break;
-    case 4: launch_moe_general<4>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, a_dt, ldo, s); break;
-    default: launch_moe_general<8>(w, tpe, A, a_dt, lda, perm, perm_div, items, n_items, max_items, out, a_dt, ldo, s);
+    case 2: launch_moe_general<2>(w, tpe, A, a_dt, lda, perm, perm_div, work, out, a_dt, ldo, s); break;
+    case 4: launch_moe_general<4>(w, tpe, A, a_dt, lda, perm, perm_div, work, out, a_dt, ldo, s); break;
+    default: launch_moe_general<8>(w, tpe, A, a_dt, lda, perm, perm_div, work, out, a_dt, ldo, s);
   }
 }
 
@@ -1293,11 +1301,10 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
   const size_t es = static_cast<size_t>(dtype_size(x_dtype));
   // Rows per work item: 64 when experts average more than 24 rows and every product takes the
   // fast path (each expert's weights are then mostly read once), else 32.
-  const int64_t inter_i = inter;
+  // (fc2's rows are the activations in the workspace, aligned.)
   const bool all_fast = moe_fast(fc1, x_dtype, d_x, static_cast<int>(T), static_cast<int>(H)) &&
                         (!two || moe_fast(fc3, x_dtype, d_x, static_cast<int>(T), static_cast<int>(H))) &&
-                        fc2->wdtype == TMH_F16 && fc2->zp_kind != TMH_ZP_FLOAT && inter_i % 8 == 0 &&
-                        tk * inter_i * 2 < (int64_t(1) << 31) && (fc2->ntiles + 1) * fc2->nchunks * 1024 < (int64_t(1) << 31);
+                        moe_fast(fc2, x_dtype, nullptr, static_cast<int>(tk), static_cast<int>(inter));
   // Few rows an expert and few experts reached (at most min(E, T k)): k_moe_rows, items of 16 rows.
   // Where more experts are reached the product that walks K reads as fast with less instruction work,
   // from fewer experts on the narrower they are (q4, us per call, this product / moe_gemm_f16, 2 to 8
@@ -1325,6 +1332,7 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
     return fail(ctx, TMH_ERR_UNSUPPORTED, "QMoE needs a %zu-byte workspace; run it once outside graph capture first", off);
   auto* n_items = reinterpret_cast<int*>(ws + o_nitems);
   auto* items = reinterpret_cast<int4*>(ws + o_items);
+  const MoeWork work{items, n_items, max_items, rows, few};
   auto* topi = reinterpret_cast<int*>(ws + o_topi);
   auto* topw = reinterpret_cast<float*>(ws + o_topw);
   auto* perm = reinterpret_cast<int*>(ws + o_perm);
@@ -1377,8 +1385,6 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
   // swiglu of fc1 and fc3 tiles, of the two halves of fc1, or an elementwise activation.
   // Interleaved swiglu pairs and the general path store the sums and activate separately.
   MoeEpilogue ep;
-  ep.rows = rows;
-  ep.few_rows = few;
   ep.bias1 = d_fc1_bias;
   ep.bias_dt = bias_dtype;
   ep.bias_ld = n1i;
@@ -1403,11 +1409,11 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
     } else {
       ep.kind = EPI_ACT;
     }
-    moe_gemm(fc1, ei, d_x, x_dtype, ti, hi, perm, ki, items, n_items, max_items, hact, inti, s, ep);
+    moe_gemm(fc1, ei, d_x, x_dtype, ti, hi, perm, ki, work, hact, inti, s, ep);
     TMH_TRY(check_launch(ctx, "k_moe_gemm (fc1)"));
   } else {
-    moe_gemm(fc1, ei, d_x, x_dtype, ti, hi, perm, ki, items, n_items, max_items, h1, n1i, s);
-    if (two) moe_gemm(fc3, ei, d_x, x_dtype, ti, hi, perm, ki, items, n_items, max_items, h3, n1i, s);
+    moe_gemm(fc1, ei, d_x, x_dtype, ti, hi, perm, ki, work, h1, n1i, s);
+    if (two) moe_gemm(fc3, ei, d_x, x_dtype, ti, hi, perm, ki, work, h3, n1i, s);
     TMH_TRY(check_launch(ctx, "k_moe_gemm (fc1)"));
     const int64_t act_n = tk * (activation == ACT_SWIGLU ? inter : n1);
     const unsigned act_grid = static_cast<unsigned>((act_n + 255) / 256);
@@ -1426,11 +1432,9 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
   // token's rows in one run; the general path keeps expert order.
   const bool fc2_fast = moe_fast(fc2, x_dtype, hact, tki, inti);
   MoeEpilogue ep2;
-  ep2.rows = rows;
-  ep2.few_rows = few;
   ep2.out_perm = fc2_fast ? perm : nullptr;
   const int* o_rows = fc2_fast ? nullptr : slot_pos;
-  moe_gemm(fc2, ei, hact, x_dtype, tki, inti, nullptr, 1, items, n_items, max_items, o, hi, s, ep2);
+  moe_gemm(fc2, ei, hact, x_dtype, tki, inti, nullptr, 1, work, o, hi, s, ep2);
   TMH_TRY(check_launch(ctx, "k_moe_gemm (fc2)"));
   // H is a multiple of 16: eight columns per thread.
   const unsigned out_grid = static_cast<unsigned>((T * H / 8 + 255) / 256);
