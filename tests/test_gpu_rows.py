@@ -27,10 +27,10 @@ def typed(x, dtype):
     return bf16_host(h) if dtype == "bf16" else h
 
 
-def check(ctx, a, a_dtype, w_dtype, k, n, bits, block, zp, bias_dtype=None, seed=0):
+def check(ctx, a, a_dtype, w_dtype, k, n, bits, block, zp, bias_dtype=None, seed=0, edit_scales=None):
     rng = np.random.default_rng(seed)
     b, s32, z = nbits_weight(rng, k, n, bits, block, zp=zp, scale_dtype=np.float32)
-    scales = typed(s32, w_dtype)
+    scales = typed(s32 if edit_scales is None else edit_scales(s32), w_dtype)
     w = PackedWeight.upload(ctx, b, scales, z, k=k, n=n, bits=bits, block_size=block, weight_dtype=w_dtype)
     bias = None if bias_dtype is None else typed(rng.standard_normal(n), bias_dtype)
     y_t = matmul_nbits(ctx.put(a), w, bias)
@@ -38,8 +38,10 @@ def check(ctx, a, a_dtype, w_dtype, k, n, bits, block, zp, bias_dtype=None, seed
     dense = o.dequantize_weight(b, as_f64(scales, w_dtype).astype(np.float32), z, k, n, bits, block, w_dtype)
     dense = np.asarray(dense, np.float64)
     af = as_f64(a, a_dtype)
-    with np.errstate(invalid="ignore"):
+    with np.errstate(invalid="ignore", over="ignore"):
         ref = af @ dense.T
+        for row in np.flatnonzero(~np.isfinite(af).all(1)) if np.isfinite(dense).all() else range(len(af)):
+            ref[row] = (af[row] * dense).sum(1)  # product by product: a matrix product may skip zeros
     dot_dtype = a_dtype if a_dtype == w_dtype else "f32"
     bound = 2.0 ** -20 * (np.abs(af) @ np.abs(dense).T) + HALF_ULP[dot_dtype] * np.abs(ref)
     if bias is not None:
@@ -106,3 +108,38 @@ def test_wide_range_infinities_and_nan(ctx, a_dtype, w_dtype):
     limit = {"f16": 65504.0}.get(a_dtype if a_dtype == w_dtype else "f32", 3.4e38)
     fits = np.abs(ref[rest]) < limit
     assert (np.abs(y[rest] - ref[rest])[fits] <= bound[rest][fits]).all()
+
+
+# Paths whose factors are cut in parts, and beside them the f16 one.
+SPECIAL = [("f32", "f16", 4, 32, "packed"), ("f16", "f32", 4, 32, "none"), ("bf16", "f32", 8, 64, "packed"),
+           ("f32", "bf16", 8, 16, "none"), ("f32", "f32", 2, 64, "packed"), ("f32", "f32", 4, 16, "none"),
+           ("f16", "f16", 4, 32, "float"), ("bf16", "bf16", 8, 32, "float"), ("f32", "f32", 8, 32, "float"),
+           ("f16", "f16", 4, 32, "packed")]
+
+
+@pytest.mark.parametrize("a_dtype,w_dtype,bits,block,zp", SPECIAL)
+@pytest.mark.parametrize("infinite_weights", [False, True])
+def test_infinities_as_in_float64(ctx, a_dtype, w_dtype, bits, block, zp, infinite_weights):
+    """An infinity or NaN in A, or an infinite weight (an f16 scale times q - zero past 65504; in the wider
+    types an infinite scale), gives +inf, -inf or NaN exactly where the float64 sum does, and every
+    finite output stays within the bound."""
+    print(f"infinities {a_dtype} {w_dtype} b{bits} bs{block} {zp} weights={infinite_weights}", flush=True)
+    rng = np.random.default_rng(6)
+    m, k, n = 20, 520, 64
+    a = np.abs(rng.standard_normal((m, k))) + 0.1
+    a[3, 17], a[4, 40], a[5, 300], a[6, 2], a[6, 500] = np.inf, -np.inf, np.nan, np.inf, -np.inf
+    a = typed(a, a_dtype)
+
+    def some_infinite(s32):
+        s = s32.reshape(n, -1).copy()
+        s[5, 1] = s[50, 0] = 60000.0 if w_dtype == "f16" else np.inf
+        return s.reshape(s32.shape)
+
+    # (f16 and bf16 operands of one type multiply on their own matrix instructions, whose weights
+    # overflow as the type does.)
+    y, ref, bound = check(ctx, a, a_dtype, w_dtype, k, n, bits, block, zp, seed=9,
+                          edit_scales=some_infinite if infinite_weights else None)
+    for kind in (np.isposinf, np.isneginf, np.isnan):
+        assert np.array_equal(kind(y), kind(ref)), kind.__name__
+    fin = np.isfinite(ref)
+    assert fin.sum() > n and (np.abs(y - ref)[fin] <= bound[fin]).all()

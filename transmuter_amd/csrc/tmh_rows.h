@@ -88,6 +88,49 @@ __device__ __noinline__ void rows_store_any(float4_t v, void* Y, uint32_t types,
   }
 }
 
+// One wavefront's sums of four consecutive columns of one row again, one f32 FMA per product as
+// k_matmul_general forms them, over its chunks c0, c0 + step, ...: for the sums that came out infinite or
+// NaN, where the parts of a factor may be at fault (0 times an infinity's other part, a weight whose
+// scale lies at the end of its type). Rare, so nothing here is made fast.
+template <int BITS>
+__device__ __forceinline__ float4_t rows_exact(const uint4_t* qt, const void* sc, const uint8_t* zp, const void* A, int a_dt,
+                                               int w_dt, uint32_t zk, uint32_t tile, uint32_t col, uint32_t a_at,
+                                               uint32_t nch, uint32_t nbc, uint32_t bsc_shift, uint32_t K, uint32_t c0,
+                                               uint32_t step) {
+  constexpr uint32_t CW = 512 / BITS, GW = CW / 4;
+  float4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (uint32_t c = c0; c < nch; c += step)
+#pragma unroll 1
+    for (uint32_t kg = 0; kg < 4; ++kg)
+#pragma unroll
+      for (uint32_t i = 0; i < GW / 8; ++i) {
+        const uint32_t kc = kg * GW + 8 * i, k = c * CW + kc;
+        if (k >= K) break;  // K is a multiple of 8
+        float a[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] = load_float_rt(A, a_dt, a_at + k + j);
+#pragma unroll 1
+        for (uint32_t e = 0; e < 4; ++e) {
+          const uint32_t at = ((tile * nch + c) * nbc + (kc >> bsc_shift)) * 16 + col + e;
+          const float s = load_float_rt(sc, w_dt, at);
+          const float z = zk == TMH_ZP_FLOAT ? reinterpret_cast<const float*>(zp)[at]
+                          : zk == TMH_ZP_PACKED
+                              ? static_cast<float>(zp_field<BITS>(zp[zp_byte<BITS>(at)], zp_shift<BITS>(static_cast<int>(col + e))))
+                              : static_cast<float>(1 << (BITS - 1));
+          float q[8], x = 0.f;
+          natural_values<BITS>(qt[(tile * nch + c) * 64 + kg * 16 + col + e], static_cast<int>(i), 1.f, 0.f, q);
+#pragma unroll
+          for (int f = 0; f < 4; ++f) x = f == static_cast<int>(e) ? sum[f] : x;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x = fmaf(round_rt(round_rt(q[j] - z, w_dt) * s, w_dt), a[j], x);
+#pragma unroll
+          for (int f = 0; f < 4; ++f) sum[f] = f == static_cast<int>(e) ? x : sum[f];
+        }
+      }
+  return sum;
+}
+
 // types = the type of Y | the dot's << 8 | the bias's << 16 (0: none) | A's << 24 (ROW_GEN); kinds =
 // the zero point kind | the weights' type << 8 (ROW_GEN). shape as in gemv_dec (M up to 64).
 // The leading arguments are preloaded into SGPRs at wave launch.
@@ -347,6 +390,30 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) rows_red[(wave * MT * TN + mt * TN + tn) * 64 + lane] = acc[mt][tn];
+  if constexpr (OP == ROW_GEN) {
+    float odd = 0.f;  // NaN where a sum is infinite or NaN, else 0
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) odd = fmaf(acc[mt][tn][e], 0.f, odd);
+    if (__builtin_expect(__any(odd != 0.f), 0)) {
+#pragma unroll 1
+      for (int p = 0; p < MT * TN; ++p) {
+        const uint32_t m = m0 + p / TN * 16 + r, tile = t0 + p % TN;
+        float4_t* const mine = rows_red + (wave * MT * TN + p) * 64 + lane;
+        const float4_t v = *mine;
+        if (m >= M || tile >= ntiles || v[0] * 0.f + v[1] * 0.f + v[2] * 0.f + v[3] * 0.f == 0.f) continue;
+        const float4_t x = rows_exact<BITS>(qt, sc, zp, A, types >> 24, (kinds >> 8) & 0xFFu, kinds & 0xFFu, tile, 4 * g,
+                                            m * lda, nch, nbc, bsc_shift, K, wave, NW);
+        float4_t out;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = v[e] * 0.f == 0.f ? v[e] : x[e];
+        *mine = out;
+      }
+    }
+  }
   __syncthreads();
   constexpr uint32_t kOwn = OP == ROW_F16 ? DT_F16 : OP == ROW_BF16 ? DT_BF16 : DT_F32;
   const bool plain = (types & 0xFFFFFFu) == (kOwn | (kOwn << 8)) && ldy % 4 == 0 &&
