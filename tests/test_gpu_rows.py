@@ -143,3 +143,31 @@ def test_infinities_as_in_float64(ctx, a_dtype, w_dtype, bits, block, zp, infini
         assert np.array_equal(kind(y), kind(ref)), kind.__name__
     fin = np.isfinite(ref)
     assert fin.sum() > n and (np.abs(y - ref)[fin] <= bound[fin]).all()
+
+
+@pytest.mark.parametrize("a_dtype,w_dtype,bits,block,zp", [("f32", "f32", 4, 16, "packed"), ("f32", "f32", 2, 64, "none"),
+                                                           ("f32", "f32", 4, 32, "float")])
+def test_parts_leave_no_bias(ctx, a_dtype, w_dtype, bits, block, zp):
+    """Both factors cut in bf16 parts, every product of one sign and significands near 2, where the
+    products of the smaller parts are largest: the mean relative error of the outputs is that of the
+    rounding of a few f32 sums (each within 2^-24, of either sign), without what a dropped product of
+    parts would take from all of them."""
+    print(f"parts {a_dtype} {w_dtype} b{bits} bs{block} {zp}", flush=True)
+    rng = np.random.default_rng(8)
+    m, k, n = 16, 16 if bits == 4 else 64, 512
+    near2 = lambda shape: (2.0 - rng.integers(1, 200, shape) * 2.0 ** -23).astype(np.float32)
+    b, s32, z = nbits_weight(rng, k, n, bits, block, zp=zp, scale_dtype=np.float32)
+    b = np.full_like(b, 0xFF)  # the largest value everywhere
+    if zp == "packed":
+        z = np.zeros_like(z)
+    elif zp == "float":
+        z = np.zeros_like(z)
+    scales, a = near2(s32.shape), near2((m, k))
+    w = PackedWeight.upload(ctx, b, scales, z, k=k, n=n, bits=bits, block_size=block, weight_dtype=w_dtype)
+    y = matmul_nbits(ctx.put(a), w).numpy().astype(np.float64)
+    w.free()
+    dense = np.asarray(o.dequantize_weight(b, scales, z, k, n, bits, block, w_dtype), np.float64)
+    ref = a.astype(np.float64) @ dense.T
+    rel = (y - ref) / ref
+    print(f"mean {rel.mean() * 2.0 ** 24:.4f} max {np.abs(rel).max() * 2.0 ** 24:.3f} units of 2^-24", flush=True)
+    assert abs(rel.mean()) <= 2.0 ** -26  # (8192 roundings of either sign average to 2^-30 and less)

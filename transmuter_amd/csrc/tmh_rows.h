@@ -24,7 +24,9 @@
 //            three MFMAs and four FMAs a lane per step, with f32 products throughout;
 //  ROW_GEN   every other combination (mixed types, float zero points, f32 weights in blocks of 16 or
 //            of 2 bits): the weights dequantize in f32 as the reference does in their type, and
-//            three bf16 parts of each factor (exact) meet in the six products above 2^-24.
+//            three bf16 parts of each factor (exact) meet in all nine products, so that none is
+//            rounded. (The parts are cut, so what the three smallest products add always has the
+//            product's own sign: left out, up to 2^-23 of each product would be missing from every sum.)
 // f16 and bf16 weights with float zero points take ROW_GEN too.
 #pragma once
 
@@ -346,7 +348,10 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
           split3(q, wp);
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) {
-            float4_t sum = mma_bf16(wp[2], ap[mt][0], float4_t{0.f, 0.f, 0.f, 0.f});
+            float4_t sum = mma_bf16(wp[2], ap[mt][2], float4_t{0.f, 0.f, 0.f, 0.f});
+            sum = mma_bf16(wp[2], ap[mt][1], sum);
+            sum = mma_bf16(wp[1], ap[mt][2], sum);
+            sum = mma_bf16(wp[2], ap[mt][0], sum);
             sum = mma_bf16(wp[1], ap[mt][1], sum);
             sum = mma_bf16(wp[0], ap[mt][2], sum);
             sum = mma_bf16(wp[1], ap[mt][0], sum);
