@@ -114,7 +114,7 @@ def test_wide_range_infinities_and_nan(ctx, a_dtype, w_dtype):
 SPECIAL = [("f32", "f16", 4, 32, "packed"), ("f16", "f32", 4, 32, "none"), ("bf16", "f32", 8, 64, "packed"),
            ("f32", "bf16", 8, 16, "none"), ("f32", "f32", 2, 64, "packed"), ("f32", "f32", 4, 16, "none"),
            ("f16", "f16", 4, 32, "float"), ("bf16", "bf16", 8, 32, "float"), ("f32", "f32", 8, 32, "float"),
-           ("f16", "f16", 4, 32, "packed")]
+           ("f16", "f16", 4, 32, "packed"), ("f32", "f32", 4, 32, "none"), ("f32", "f32", 8, 64, "packed")]
 
 
 @pytest.mark.parametrize("a_dtype,w_dtype,bits,block,zp", SPECIAL)
@@ -171,3 +171,18 @@ def test_parts_leave_no_bias(ctx, a_dtype, w_dtype, bits, block, zp):
     rel = (y - ref) / ref
     print(f"mean {rel.mean() * 2.0 ** 24:.4f} max {np.abs(rel).max() * 2.0 ** 24:.3f} units of 2^-24", flush=True)
     assert abs(rel.mean()) <= 2.0 ** -26  # (8192 roundings of either sign average to 2^-30 and less)
+
+
+@pytest.mark.parametrize("bits,block,zp", [(4, 32, "none"), (4, 128, "packed"), (8, 32, "packed"), (8, 64, "none")])
+def test_f32_a_near_the_end_of_its_range(ctx, bits, block, zp):
+    """A up to 3e38 against small scales: every output is finite, also where the products of a block
+    pass f32's range before its scale."""
+    print(f"range b{bits} bs{block} {zp}", flush=True)
+    rng = np.random.default_rng(12)
+    m, k, n = 20, 520, 80
+    a = rng.standard_normal((m, k)) * 10.0 ** rng.uniform(33, 37.8, (m, 1))
+    a[7] = 3e38  # one sign: every block's sum is past the range
+    a = np.clip(a, -3e38, 3e38).astype(np.float32)
+    y, ref, bound = check(ctx, a, "f32", "f32", k, n, bits, block, zp, seed=3, edit_scales=lambda s: s * np.float32(1e-4))
+    assert np.isfinite(ref).all() and np.abs(ref).max() < 3e38
+    assert (np.abs(y - ref) <= bound).all()

@@ -21,7 +21,9 @@
 //  ROW_INT   f32 A and f32 weights of blocks of 32 and more: q - zero is a whole number of at most
 //            8 bits and so exact in bf16, a value of A is the exact sum of three bf16 parts, and a
 //            step's 32 products sit in one block, whose f32 scale multiplies the step's f32 sums:
-//            three MFMAs and four FMAs a lane per step, with f32 products throughout;
+//            three MFMAs and four FMAs a lane per step, with f32 products throughout. (A step's sum
+//            before its scale can pass f32's range, from |a| near 4e34 with 8 bits and 7e35 with 4
+//            on: it comes out infinite or NaN then, and rows_exact forms the sums again.);
 //  ROW_GEN   every other combination (mixed types, float zero points, f32 weights in blocks of 16 or
 //            of 2 bits): the weights dequantize in f32 as the reference does in their type, and
 //            three bf16 parts of each factor (exact) meet in all nine products, so that none is
@@ -41,21 +43,15 @@ typedef __bf16 rows_bf16x8_t __attribute__((ext_vector_type(8)));
 
 // Eight f32 values as the sum of three bf16 parts each: the top 8 bits of the significand, the next
 // 8 and the last 8 (cut, not rounded: every part is exact, and no part of a finite value
-// overflows). An infinity is its first part; what is left of it (inf - inf) counts as 0.
+// overflows; below 2^-110 the last bits fall under bf16's own range). An infinity leaves a NaN
+// behind: the sums it enters are formed again (rows_exact).
 __device__ __forceinline__ void split3(const float (&a)[8], uint4_t (&part)[3]) {
   float rest[8];
   uint32_t top[8];
-  float big = 0.f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     top[j] = __builtin_bit_cast(uint32_t, a[j]);
     rest[j] = a[j] - __builtin_bit_cast(float, top[j] & 0xFFFF0000u);
-    big = fmaxf(big, fabsf(a[j]));
-  }
-  if (__builtin_expect(__any(big == INFINITY), 0)) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (fabsf(a[j]) == INFINITY) rest[j] = 0.f;
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -395,7 +391,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) rows_red[(wave * MT * TN + mt * TN + tn) * 64 + lane] = acc[mt][tn];
-  if constexpr (OP == ROW_GEN) {
+  if constexpr (OP == ROW_GEN || OP == ROW_INT) {
     float odd = 0.f;  // NaN where a sum is infinite or NaN, else 0
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
