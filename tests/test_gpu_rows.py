@@ -114,7 +114,8 @@ def test_wide_range_infinities_and_nan(ctx, a_dtype, w_dtype):
 SPECIAL = [("f32", "f16", 4, 32, "packed"), ("f16", "f32", 4, 32, "none"), ("bf16", "f32", 8, 64, "packed"),
            ("f32", "bf16", 8, 16, "none"), ("f32", "f32", 2, 64, "packed"), ("f32", "f32", 4, 16, "none"),
            ("f16", "f16", 4, 32, "float"), ("bf16", "bf16", 8, 32, "float"), ("f32", "f32", 8, 32, "float"),
-           ("f16", "f16", 4, 32, "packed"), ("f32", "f32", 4, 32, "none"), ("f32", "f32", 8, 64, "packed")]
+           ("f16", "f16", 4, 32, "packed"), ("f32", "f32", 4, 32, "none"), ("f32", "f32", 8, 64, "packed"),
+           ("bf16", "bf16", 4, 32, "packed"), ("bf16", "bf16", 2, 64, "none")]
 
 
 @pytest.mark.parametrize("a_dtype,w_dtype,bits,block,zp", SPECIAL)
@@ -185,4 +186,20 @@ def test_f32_a_near_the_end_of_its_range(ctx, bits, block, zp):
     a = np.clip(a, -3e38, 3e38).astype(np.float32)
     y, ref, bound = check(ctx, a, "f32", "f32", k, n, bits, block, zp, seed=3, edit_scales=lambda s: s * np.float32(1e-4))
     assert np.isfinite(ref).all() and np.abs(ref).max() < 3e38
+    assert (np.abs(y - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("bits,block,zp", [(4, 32, "packed"), (4, 16, "none"), (8, 64, "none"), (2, 64, "packed")])
+@pytest.mark.parametrize("power", [-132, -120, 117])
+def test_bf16_scales_at_the_ends_of_the_type(ctx, bits, block, zp, power):
+    """bf16 scales of 2^117 to 2^120, and subnormal and nearly subnormal ones, against A at the other
+    end of the type."""
+    print(f"bf16 scales 2^{power} b{bits} bs{block} {zp}", flush=True)
+    rng = np.random.default_rng(13)
+    m, k, n = 20, 264, 80
+    a = typed(rng.standard_normal((m, k)) * 2.0 ** (100 if power < 0 else -100), "bf16")
+    edit = lambda s: (rng.uniform(1, 8, s.shape) * 2.0 ** power).astype(np.float32)
+    y, ref, bound = check(ctx, a, "bf16", "bf16", k, n, bits, block, zp, seed=4, edit_scales=edit)
+    assert np.isfinite(ref).all()
+    print(f"largest error over its bound {(np.abs(y - ref) / bound).max():.3f}", flush=True)
     assert (np.abs(y - ref) <= bound).all()

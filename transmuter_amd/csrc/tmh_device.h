@@ -246,7 +246,8 @@ __device__ __forceinline__ void natural_params(uint32_t x, uint32_t* out) {
 // scale * (q - zero) of the eight values q of step i, in k order: one fma each over the f16 numbers
 // 1024 + q that the packed values become under the exponent of 0x6400 (as in unpack_step; the
 // nibbles at bits 4-7 give 1024 + 16 q, whose scale is scale / 16). Each product and sum is exact
-// (for a bf16 scale below 2^117, or scale 1), so the fma's one rounding rounds nothing.
+// (for a bf16 scale below 2^117, or scale 1; from there on the offset of 1024 can overflow and the
+// values come out infinite or NaN), so the fma's one rounding rounds nothing.
 template <int BITS>
 __device__ __forceinline__ void natural_values(const uint4_t& w, int i, float scale, float zero, float (&q)[8]) {
   // (Held from constant folding: a scale of 1 known to the compiler becomes a conversion and a

@@ -17,7 +17,8 @@
 // Operand paths (OP):
 //  ROW_F16   f16 A and weights: exact f16 weights (q - zero) * scale (unpack_step);
 //  ROW_BF16  bf16 A and weights: (q - zero) * scale formed in f32 and rounded once to bf16, as the
-//            reference's bf16 dequantization rounds it;
+//            reference's bf16 dequantization rounds it (a scale of 2^117 and more overflows on the way,
+//            natural_values: rows_exact forms the sums of such weights);
 //  ROW_INT   f32 A and f32 weights of blocks of 32 and more: q - zero is a whole number of at most
 //            8 bits and so exact in bf16, a value of A is the exact sum of three bf16 parts, and a
 //            step's 32 products sit in one block, whose f32 scale multiplies the step's f32 sums:
@@ -391,7 +392,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) rows_red[(wave * MT * TN + mt * TN + tn) * 64 + lane] = acc[mt][tn];
-  if constexpr (OP == ROW_GEN || OP == ROW_INT) {
+  if constexpr (OP != ROW_F16) {
     float odd = 0.f;  // NaN where a sum is infinite or NaN, else 0
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
