@@ -203,3 +203,26 @@ def test_bf16_scales_at_the_ends_of_the_type(ctx, bits, block, zp, power):
     assert np.isfinite(ref).all()
     print(f"largest error over its bound {(np.abs(y - ref) / bound).max():.3f}", flush=True)
     assert (np.abs(y - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("bits,block,zp", [(4, 32, "none"), (4, 128, "packed"), (8, 32, "packed"), (8, 64, "none")])
+@pytest.mark.parametrize("m,k,n", [(70, 520, 80), (100, 2048, 300)])
+def test_prefill_f32_over_a_s_whole_range(ctx, bits, block, zp, m, k, n):
+    """The f32 prefill product (over 64 rows, whole-number weights): A up to 3e38 against small scales
+    gives finite outputs, A down to 1e-30 the same relative error, and an infinity or a NaN in a row of A
+    what the float64 sum gives. A's hi and lo parts hold 16 bits of each value: 2^-16 of every product."""
+    print(f"prefill range b{bits} bs{block} {zp} m={m}", flush=True)
+    rng = np.random.default_rng(14)
+    a = rng.standard_normal((m, k)) * 10.0 ** rng.uniform(-30, 37.8, (m, 1))
+    a[7] = 3e38  # one sign: every block's sum is past the range before its scale
+    a = np.clip(a, -3e38, 3e38).astype(np.float32)
+    a[66] = np.abs(a[66]) + 1.0
+    a[66, 3] = np.inf
+    a[67, 5] = np.nan
+    y, ref, bound = check(ctx, a, "f32", "f32", k, n, bits, block, zp, seed=3, edit_scales=lambda s: s * np.float32(1e-4))
+    for kind in (np.isposinf, np.isneginf, np.isnan):
+        assert np.array_equal(kind(y), kind(ref)), kind.__name__
+    fin = np.isfinite(ref).all(1)
+    assert fin.sum() == m - 2 and np.abs(ref[fin]).max() < 3e38
+    # bound holds 2^-20 sum |a w|: 16 times that is 2^-16 of every product
+    assert (np.abs(y - ref)[fin] <= 16 * bound[fin]).all()

@@ -391,10 +391,15 @@ constexpr int kGemmBM = 256;  // largest tile height: bounds the A rows a launch
 //           bf16; the weight words trade lanes (natural_words) so that a step's 32 values of k lie in
 //           one block, and the block's f32 scale multiplies the step's f32 sums: two MFMAs per product
 //           (the hi and lo rows of A) and four FMAs a lane, in place of three MFMAs and the splitting
-//           of every weight, and no rounding of the weights. 509 x 1024 -> 6144 (kernel alone, traced):
+//           of every weight, and no rounding of the weights. They enter as (q - zero) times 2^-9 (4
+//           bits) or 2^-13 (8 bits), exact too, so that no block's sum passes A's own range before its
+//           scale, and the sums take the power back at the end: full precision down to outputs of 1e-35. 509 x 1024 -> 6144 (kernel alone, traced):
 //           32.3 -> 27.3 us; the four projections of a layer of that width, with the splitting of A and
 //           the split-K sums, 121.6 -> 97.5 us; relative error against float64 4.5e-6 -> 2.5e-6.
 enum : int { GM_F16 = 0, GM_BF16 = 1, GM_SPLIT = 2, GM_INT = 3 };
+// What GM_INT's sums are multiplied by at the end: above 32 times the largest |q - zero|.
+template <int BITS>
+constexpr float kIntGrow = BITS == 8 ? 8192.f : 512.f;
 // The paths that take A as hi and lo rows of bf16.
 constexpr bool splits_a(int mode) { return mode == GM_SPLIT || mode == GM_INT; }
 
@@ -716,6 +721,7 @@ __device__ __forceinline__ void gemm_lds(
   auto compute = [&](int buf, const BStage& st, bool more, uint32_t kbn, BStage& nst) {
     const uint8_t* abase = lds + buf * ABUF + (wm * 128 + r) * ROWB;
     if constexpr (MODE == GM_INT) {
+      constexpr float kShrink = 1.f / kIntGrow<BITS>;
       uint4_t wn[NTW];
       uint32_t zn[NTW][STEPS];
 #pragma unroll
@@ -734,7 +740,7 @@ __device__ __forceinline__ void gemm_lds(
 #pragma unroll
           for (int nt = 0; nt < NTW; ++nt) {
             float q[8];
-            natural_values<BITS>(wn[nt], i, 1.f, static_cast<float>(zn[nt][i]), q);
+            natural_values<BITS>(wn[nt], i, kShrink, static_cast<float>(zn[nt][i]), q);
 #pragma unroll
             for (int j = 0; j < 4; ++j) b[nt][j] = pack_bf16_rne(q[2 * j], q[2 * j + 1]);
           }
@@ -915,6 +921,12 @@ __device__ __forceinline__ void gemm_lds(
     }
     __syncthreads();
     if (more) cur = next;
+  }
+  if constexpr (MODE == GM_INT) {
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NTW; ++nt) acc[mt][nt] *= kIntGrow<BITS>;
   }
   if constexpr (KS == 2) {
     // The second half's partial sums through LDS (free after the k-loop's last barrier: no
