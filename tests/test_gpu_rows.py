@@ -226,3 +226,16 @@ def test_prefill_f32_over_a_s_whole_range(ctx, bits, block, zp, m, k, n):
     assert fin.sum() == m - 2 and np.abs(ref[fin]).max() < 3e38
     # bound holds 2^-20 sum |a w|: 16 times that is 2^-16 of every product
     assert (np.abs(y - ref)[fin] <= 16 * bound[fin]).all()
+
+
+# Over 64 rows without a build of the prefill GEMM: slices of 64 rows in one launch, the rest in a second.
+@pytest.mark.parametrize("a_dtype,w_dtype,bits,block,zp", [("bf16", "bf16", 4, 16, "packed"), ("f32", "f32", 4, 16, "none"),
+                                                           ("f32", "f16", 2, 32, "packed"), ("f16", "f16", 2, 16, "float")])
+@pytest.mark.parametrize("m,n", [(65, 48), (128, 20), (129, 300), (1000, 64)])
+def test_slices_of_64_rows(ctx, m, n, a_dtype, w_dtype, bits, block, zp):
+    print(f"slices m={m} n={n} {a_dtype} {w_dtype} b{bits} bs{block} {zp}", flush=True)
+    rng = np.random.default_rng(m + n)
+    k = chunk(bits) + 40
+    a = typed(rng.standard_normal((m, k)), a_dtype)
+    y, ref, bound = check(ctx, a, a_dtype, w_dtype, k, n, bits, block, zp, "f32" if m == 129 else None, seed=n)
+    assert (np.abs(y - ref) <= bound).all()

@@ -2244,12 +2244,8 @@ int launch_matmul(tmh_ctx* ctx, const tmh_weight* w, const MatArgs& a, hipStream
   }
   if ((a.M <= 64 || !fast_path(w, a)) && gemv_rows_ok(w, a.a, a.a_dt, std::min<int64_t>(a.M, 64), a.lda)) {
     // (More than 64 rows come here where the GEMM has no build for the parameters, bf16 or f32 with
-    // several blocks in a lane's group, or no 32-bit offsets over A: in launches of 64 rows.)
-    for (int64_t m = 0; m < a.M; m += 64)
-      launch_gemv_rows(w, static_cast<const uint8_t*>(a.a) + m * a.lda * dtype_size(a.a_dt), a.a_dt,
-                       std::min<int64_t>(a.M - m, 64), a.lda, a.bias, a.bias_dt,
-                       static_cast<uint8_t*>(a.y) + m * a.ldy * dtype_size(a.y_dt), a.y_dt, a.dot_dt, a.ldy, s,
-                       ctx->num_cus);
+    // several blocks in a lane's group, or no 32-bit offsets over A.)
+    launch_gemv_rows(w, a.a, a.a_dt, a.M, a.lda, a.bias, a.bias_dt, a.y, a.y_dt, a.dot_dt, a.ldy, s, ctx->num_cus);
     return check_launch(ctx, "k_gemv_rows");
   }
   if (fast_path(w, a)) {

@@ -131,12 +131,13 @@ __device__ __forceinline__ float4_t rows_exact(const uint4_t* qt, const void* sc
 }
 
 // types = the type of Y | the dot's << 8 | the bias's << 16 (0: none) | A's << 24 (ROW_GEN); kinds =
-// the zero point kind | the weights' type << 8 (ROW_GEN). shape as in gemv_dec (M up to 64).
+// the zero point kind | the weights' type << 8 (ROW_GEN). shape as in gemv_dec (M up to 64). Workgroups of
+// blockIdx.z = s take rows 64 s to 64 s + M of A and Y.
 // The leading arguments are preloaded into SGPRs at wave launch.
 template <int BITS, int OP, bool SPLIT, int MT, int TN, int NW>
 __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
     const uint4_t* __restrict__ qt, const void* __restrict__ sc, const uint8_t* __restrict__ zp,
-    const void* __restrict__ A, uint32_t nch, uint32_t ntiles, uint32_t lda, uint32_t shape, void* __restrict__ Y,
+    const void* __restrict__ a, uint32_t nch, uint32_t ntiles, uint32_t lda, uint32_t shape, void* __restrict__ Y,
     int64_t ldy, uint32_t N, uint32_t types, uint32_t kinds, const void* __restrict__ bias) {
   constexpr int CW = 512 / BITS;
   constexpr int GW = CW / 4;
@@ -168,6 +169,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
   // (Without zero points the resource is empty and its loads read zeros, not used.)
   const auto z_rsrc = buffer_rsrc(zp, zk == TMH_ZP_NONE ? 0u : zk == TMH_ZP_FLOAT ? n_params * 4 : zp_byte<BITS>(n_params));
   const uint32_t zsh = zp_shift<BITS>(r);
+  const void* const A = static_cast<const uint8_t*>(a) + static_cast<uint64_t>(blockIdx.z) * (64 * lda * a_size);
   const auto a_rsrc = buffer_rsrc(A, M * lda * a_size);
   uint32_t a_row[MT];
 #pragma unroll
@@ -434,7 +436,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
     float4_t v = part[0];
 #pragma unroll
     for (int w2 = 1; w2 < NW; ++w2) v += part[w2];
-    const int64_t at = static_cast<int64_t>(m) * ldy + n;
+    const int64_t at = (static_cast<int64_t>(blockIdx.z) * 64 + m) * ldy + n;
     if (plain && n + 4 <= N) {  // Y in the operands' own type, no bias
       if constexpr (OP == ROW_F16) {
         const half2_t lo = {static_cast<_Float16>(v[0]), static_cast<_Float16>(v[1])};
