@@ -341,8 +341,17 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
           const float z = zk == TMH_ZP_FLOAT ? __builtin_bit_cast(float, zraw) : static_cast<float>(zero_of(zraw));
           float q[8];
           natural_values<BITS>(st.w[tn], i, 1.f, 0.f, q);  // q itself: a float zero point is subtracted as it is
+          // (One uniform branch over the type a step, not two a value.)
+          if (w_dt == DT_F32) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) q[e] = round_rt(round_rt(q[e] - z, w_dt) * s, w_dt);
+            for (int e = 0; e < 8; ++e) q[e] = (q[e] - z) * s;
+          } else if (w_dt == DT_F16) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) q[e] = round_to<DT_F16>(round_to<DT_F16>(q[e] - z) * s);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) q[e] = round_to<DT_BF16>(round_to<DT_BF16>(q[e] - z) * s);
+          }
           uint4_t wp[3];
           split3(q, wp);
 #pragma unroll
