@@ -118,9 +118,9 @@ bool decode_gemv_f32_ok(const tmh_weight* w, int64_t M, int64_t lda, int64_t ldy
 void launch_decode_gemv_f32(const tmh_weight* w, const void* a, int64_t M, int64_t lda, void* y, int64_t ldy,
                             hipStream_t s);
 
-// The products of up to 64 rows of A in any float types, and of more in slices of 64 (k_gemv_rows,
-// tmh_rows.hip). gemv_rows_ok tells whether the kernel applies to M rows (aligned rows of A, K a
-// multiple of 8, 32-bit offsets); for more than 64 it is asked about one slice.
+// The products of up to 64 rows of A in any float types, and of more where no other kernel is built for
+// the types (k_gemv_rows, tmh_rows.hip). gemv_rows_ok tells whether the kernel applies to M rows, up to 64
+// (aligned rows of A, K a multiple of 8, 32-bit offsets); for more it is asked about 64 of them.
 bool gemv_rows_ok(const tmh_weight* w, const void* a, int a_dtype, int64_t M, int64_t lda);
 void launch_gemv_rows(const tmh_weight* w, const void* a, int a_dtype, int64_t M, int64_t lda, const void* bias,
                       int bias_dtype, void* y, int y_dtype, int dot_dtype, int64_t ldy, hipStream_t s, int num_cus);

@@ -40,6 +40,8 @@ namespace tmh {
 
 enum : int { ROW_F16 = 0, ROW_BF16 = 1, ROW_INT = 2, ROW_GEN = 3 };
 
+constexpr int64_t kRowsMax = 4032;  // rows of A of one launch: 12 bits of its shape, in sets of 64
+
 typedef __bf16 rows_bf16x8_t __attribute__((ext_vector_type(8)));
 
 // Eight f32 values as the sum of three bf16 parts each: the top 8 bits of the significand, the next
@@ -131,13 +133,13 @@ __device__ __forceinline__ float4_t rows_exact(const uint4_t* qt, const void* sc
 }
 
 // types = the type of Y | the dot's << 8 | the bias's << 16 (0: none) | A's << 24 (ROW_GEN); kinds =
-// the zero point kind | the weights' type << 8 (ROW_GEN). shape as in gemv_dec (M up to 64). Workgroups of
-// blockIdx.z = s take rows 64 s to 64 s + M of A and Y.
+// the zero point kind | the weights' type << 8 (ROW_GEN). shape = M (up to
+// kRowsMax) | nbc << 12 | the shift of a block's k in its chunk << 20 | the eights of the last chunk past K << 24.
 // The leading arguments are preloaded into SGPRs at wave launch.
 template <int BITS, int OP, bool SPLIT, int MT, int TN, int NW>
 __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
     const uint4_t* __restrict__ qt, const void* __restrict__ sc, const uint8_t* __restrict__ zp,
-    const void* __restrict__ a, uint32_t nch, uint32_t ntiles, uint32_t lda, uint32_t shape, void* __restrict__ Y,
+    const void* __restrict__ A, uint32_t nch, uint32_t ntiles, uint32_t lda, uint32_t shape, void* __restrict__ Y,
     int64_t ldy, uint32_t N, uint32_t types, uint32_t kinds, const void* __restrict__ bias) {
   constexpr int CW = 512 / BITS;
   constexpr int GW = CW / 4;
@@ -151,8 +153,8 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
   static_assert(OP != ROW_INT || (!SPLIT && NAT), "one block per step");
   static_assert(NW * MT * TN <= 128, "the partial sums must fit the LDS");
   extern __shared__ float4_t rows_red[];
-  const uint32_t M = shape & 0xFFu, nbc = (shape >> 8) & 0xFFu, bsc_shift = (shape >> 16) & 0xFFu;
-  const uint32_t K = nch * CW - (shape >> 24) * 4;
+  const uint32_t M = shape & 0xFFFu, nbc = (shape >> 12) & 0xFFu, bsc_shift = (shape >> 20) & 0xFu;
+  const uint32_t K = nch * CW - ((shape >> 24) & 0x7Fu) * 8;
   const int lane = threadIdx.x & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -169,7 +171,6 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
   // (Without zero points the resource is empty and its loads read zeros, not used.)
   const auto z_rsrc = buffer_rsrc(zp, zk == TMH_ZP_NONE ? 0u : zk == TMH_ZP_FLOAT ? n_params * 4 : zp_byte<BITS>(n_params));
   const uint32_t zsh = zp_shift<BITS>(r);
-  const void* const A = static_cast<const uint8_t*>(a) + static_cast<uint64_t>(blockIdx.z) * (64 * lda * a_size);
   const auto a_rsrc = buffer_rsrc(A, M * lda * a_size);
   uint32_t a_row[MT];
 #pragma unroll
@@ -445,7 +446,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
     float4_t v = part[0];
 #pragma unroll
     for (int w2 = 1; w2 < NW; ++w2) v += part[w2];
-    const int64_t at = (static_cast<int64_t>(blockIdx.z) * 64 + m) * ldy + n;
+    const int64_t at = static_cast<int64_t>(m) * ldy + n;
     if (plain && n + 4 <= N) {  // Y in the operands' own type, no bias
       if constexpr (OP == ROW_F16) {
         const half2_t lo = {static_cast<_Float16>(v[0]), static_cast<_Float16>(v[1])};

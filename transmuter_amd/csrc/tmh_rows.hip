@@ -24,21 +24,21 @@ struct RowsPlan {
 };
 
 template <int BITS, int OP, bool SPLIT, int MT, int TN, int NW>
-void go_rows(const RowsArgs& d, int64_t M, unsigned slices, hipStream_t s) {
+void go_rows(const RowsArgs& d, int64_t M, hipStream_t s) {
   constexpr int kLds = NW * MT * TN * 1024;
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemv_rows<BITS, OP, SPLIT, MT, TN, NW>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   (void)attr;
-  const dim3 grid((d.ntiles + TN - 1) / TN, static_cast<unsigned>((M + 16 * MT - 1) / (16 * MT)), slices);
+  const dim3 grid((d.ntiles + TN - 1) / TN, static_cast<unsigned>((M + 16 * MT - 1) / (16 * MT)));
   k_gemv_rows<BITS, OP, SPLIT, MT, TN, NW><<<grid, 64 * NW, kLds, s>>>(d.qt, d.sc, d.zp, d.a, d.nch, d.ntiles, d.lda,
                                                                        d.shape, d.y, d.ldy, d.n, d.types, d.kinds, d.bias);
 }
 
 // The shapes plan_rows() chooses from, per operand path.
 template <int BITS, int OP, bool SPLIT>
-void launch_op(const RowsArgs& d, int64_t M, unsigned slices, const RowsPlan& p, hipStream_t s) {
+void launch_op(const RowsArgs& d, int64_t M, const RowsPlan& p, hipStream_t s) {
 #define TMH_ROWS(MT_, TN_, NW_) \
-  if (p.mt == MT_ && p.tn == TN_ && p.nw == NW_) return go_rows<BITS, OP, SPLIT, MT_, TN_, NW_>(d, M, slices, s)
+  if (p.mt == MT_ && p.tn == TN_ && p.nw == NW_) return go_rows<BITS, OP, SPLIT, MT_, TN_, NW_>(d, M, s)
   if constexpr (OP != ROW_GEN) {
     TMH_ROWS(1, 2, 8);
     TMH_ROWS(2, 2, 8);
@@ -52,7 +52,7 @@ void launch_op(const RowsArgs& d, int64_t M, unsigned slices, const RowsPlan& p,
       }
     }
   }
-  go_rows<BITS, OP, SPLIT, 1, 1, 8>(d, M, slices, s);
+  go_rows<BITS, OP, SPLIT, 1, 1, 8>(d, M, s);
 #undef TMH_ROWS
 }
 
@@ -112,10 +112,8 @@ bool gemv_rows_ok(const tmh_weight* w, const void* a, int a_dtype, int64_t M, in
 
 namespace {
 
-// `slices` sets of M rows (more than one only of 64 rows), one after the other in A and Y.
-void launch_slices(const tmh_weight* w, const void* a, int a_dtype, int64_t M, unsigned slices, int64_t lda,
-                   const void* bias, int bias_dtype, void* y, int y_dtype, int dot_dtype, int64_t ldy, hipStream_t s,
-                   int num_cus) {
+void launch_rows(const tmh_weight* w, const void* a, int a_dtype, int64_t M, int64_t lda, const void* bias, int bias_dtype,
+                 void* y, int y_dtype, int dot_dtype, int64_t ldy, hipStream_t s, int num_cus) {
   const int cw = chunk_weights(w->bits);
   int shift = 0;
   while ((1 << shift) < std::min(w->block_size, cw)) ++shift;
@@ -124,26 +122,26 @@ void launch_slices(const tmh_weight* w, const void* a, int a_dtype, int64_t M, u
   const uint32_t pad = static_cast<uint32_t>((w->nchunks * cw - w->K) / 4);
   const RowsArgs d{reinterpret_cast<const uint4_t*>(w->d_q), w->d_scale, static_cast<const uint8_t*>(w->d_zero), a,
                    static_cast<uint32_t>(w->nchunks), static_cast<uint32_t>(w->ntiles), static_cast<uint32_t>(lda),
-                   static_cast<uint32_t>(M) | (static_cast<uint32_t>(w->nbc) << 8) | (static_cast<uint32_t>(shift) << 16) | (pad << 24),
+                   static_cast<uint32_t>(M) | (static_cast<uint32_t>(w->nbc) << 12) | (static_cast<uint32_t>(shift) << 20) | (pad / 2 << 24),
                    y, ldy, static_cast<uint32_t>(w->N),
                    static_cast<uint32_t>(y_dtype) | (static_cast<uint32_t>(dot_dtype) << 8) |
                        (static_cast<uint32_t>(bias ? bias_dtype : 0) << 16) | (static_cast<uint32_t>(a_dtype) << 24),
                    static_cast<uint32_t>(w->zp_kind) | (static_cast<uint32_t>(w->wdtype) << 8), bias};
-  const RowsPlan p = plan_rows(op, w->bits == 2 || split, M * slices, w->ntiles, w->nchunks, num_cus > 0 ? num_cus : 256);
+  const RowsPlan p = plan_rows(op, w->bits == 2 || split, M, w->ntiles, w->nchunks, num_cus > 0 ? num_cus : 256);
 #define TMH_ROWS_BITS(B)                                                          \
   switch (op) {                                                                   \
     case ROW_F16:                                                                 \
-      if (split) launch_op<B, ROW_F16, true>(d, M, slices, p, s);                         \
-      else launch_op<B, ROW_F16, false>(d, M, slices, p, s);                              \
+      if (split) launch_op<B, ROW_F16, true>(d, M, p, s);                         \
+      else launch_op<B, ROW_F16, false>(d, M, p, s);                              \
       break;                                                                      \
     case ROW_BF16:                                                                \
-      if (split) launch_op<B, ROW_BF16, true>(d, M, slices, p, s);                        \
-      else launch_op<B, ROW_BF16, false>(d, M, slices, p, s);                             \
+      if (split) launch_op<B, ROW_BF16, true>(d, M, p, s);                        \
+      else launch_op<B, ROW_BF16, false>(d, M, p, s);                             \
       break;                                                                      \
     case ROW_INT:                                                                 \
-      if constexpr (B != 2) launch_op<B, ROW_INT, false>(d, M, slices, p, s);             \
+      if constexpr (B != 2) launch_op<B, ROW_INT, false>(d, M, p, s);             \
       break;                                                                      \
-    default: launch_op<B, ROW_GEN, true>(d, M, slices, p, s);                             \
+    default: launch_op<B, ROW_GEN, true>(d, M, p, s);                             \
   }
   switch (w->bits) {
     case 2: TMH_ROWS_BITS(2) break;
@@ -155,19 +153,16 @@ void launch_slices(const tmh_weight* w, const void* a, int a_dtype, int64_t M, u
 
 }  // namespace
 
-// More than 64 rows in slices of 64, all of one launch, and the rest in a second: each slice reads all
-// of the weights, but a slice alone would leave the chip idle where N is small (bf16 in blocks of 16, us:
-// 16384 x 64 -> 64 k_matmul_general 218, a launch a slice 516, this 9.3; 1024 x 2048 -> 2048 2390, 93, 53).
+// As many rows a launch as its shape and 32-bit offsets over A take: a launch for every 64 rows would
+// leave the chip idle where N is small (bf16 in blocks of 16, us: 16384 x 64 -> 64 k_matmul_general 218,
+// a launch for every 64 rows 516, this 14.5; 1024 x 2048 -> 2048 2390, 93, 53).
 void launch_gemv_rows(const tmh_weight* w, const void* a, int a_dtype, int64_t M, int64_t lda, const void* bias,
                       int bias_dtype, void* y, int y_dtype, int dot_dtype, int64_t ldy, hipStream_t s, int num_cus) {
-  constexpr int64_t kSlices = 1 << 14;  // of one launch at most
-  for (int64_t m = 0; m < M;) {
-    const int64_t slices = std::min(kSlices, (M - m) / 64), rows = slices ? 64 : M - m;
-    launch_slices(w, static_cast<const uint8_t*>(a) + m * lda * dtype_size(a_dtype), a_dtype, rows,
-                  slices ? static_cast<unsigned>(slices) : 1u, lda, bias, bias_dtype,
-                  static_cast<uint8_t*>(y) + m * ldy * dtype_size(y_dtype), y_dtype, dot_dtype, ldy, s, num_cus);
-    m += slices ? slices * 64 : rows;
-  }
+  const int64_t a_size = dtype_size(a_dtype), fit = ((int64_t(1) << 31) - 1) / (lda * a_size) / 64 * 64;
+  const int64_t most = std::max<int64_t>(64, std::min(kRowsMax, fit));  // (gemv_rows_ok: M or 64 rows fit)
+  for (int64_t m = 0; m < M; m += most)
+    launch_rows(w, static_cast<const uint8_t*>(a) + m * lda * a_size, a_dtype, std::min(most, M - m), lda, bias, bias_dtype,
+                static_cast<uint8_t*>(y) + m * ldy * dtype_size(y_dtype), y_dtype, dot_dtype, ldy, s, num_cus);
 }
 
 }  // namespace tmh
