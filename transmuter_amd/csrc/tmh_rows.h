@@ -77,15 +77,48 @@ __device__ __forceinline__ float round_rt(float x, int dt) {
 }
 
 // Four consecutive outputs at element `at` (columns n.., those below N) in any float type: the dot
-// type's rounding, then the bias. Out of line: the uniform branches over the types cost the common
-// stores nothing.
-__device__ __noinline__ void rows_store_any(float4_t v, void* Y, uint32_t types, const void* bias, int64_t at, uint32_t n,
-                                            uint32_t N) {
+// type's rounding, then the columns' bias (its bits b); in one store where Y is aligned (vec). Out of line: the
+// uniform branches over the types cost the common stores nothing.
+__device__ __noinline__ void rows_store_any(float4_t v, void* Y, uint32_t types, uint4_t b, int64_t at, uint32_t n,
+                                            uint32_t N, bool vec) {
   const int y_dt = types & 0xFFu, dot_dt = (types >> 8) & 0xFFu, b_dt = (types >> 16) & 0xFFu;
-  for (uint32_t e = 0; e < 4 && n + e < N; ++e) {
-    float x = round_rt(v[e], dot_dt);
-    if (b_dt) x += load_float_rt(bias, b_dt, n + e);
-    store_float_rt(Y, y_dt, at + e, x);
+  if (dot_dt == DT_F16) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = round_to<DT_F16>(v[e]);
+  } else if (dot_dt == DT_BF16) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = round_to<DT_BF16>(v[e]);
+  }
+  if (b_dt) {
+    float4_t f = __builtin_bit_cast(float4_t, b);  // whole vector: hipcc 7.2 miscompiled element casts
+    if (b_dt != DT_F32) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        f[e] = b_dt == DT_F16 ? f16_bits_to_f32(static_cast<uint16_t>(b[e])) : bf16_bits_to_f32(static_cast<uint16_t>(b[e]));
+    }
+    v += f;
+  }
+  if (y_dt == DT_F32) {
+    float* y = static_cast<float*>(Y) + at;
+    if (vec && n + 4 <= N) {
+      *reinterpret_cast<float4_t*>(y) = v;
+    } else {
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e)
+        if (n + e < N) y[e] = v[e];
+    }
+    return;
+  }
+  uint16_t h[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) h[e] = y_dt == DT_F16 ? f32_to_f16_bits(v[e]) : f32_to_bf16_bits(v[e]);
+  uint16_t* y = static_cast<uint16_t*>(Y) + at;
+  if (vec && n + 4 <= N) {
+    *reinterpret_cast<uint2*>(y) = make_uint2(h[0] | (static_cast<uint32_t>(h[1]) << 16), h[2] | (static_cast<uint32_t>(h[3]) << 16));
+  } else {
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e)
+      if (n + e < N) y[e] = h[e];
   }
 }
 
@@ -135,7 +168,8 @@ __device__ __noinline__ float4_t rows_exact(const uint4_t* qt, const void* sc, c
 
 // types = the type of Y | the dot's << 8 | the bias's << 16 (0: none) | A's << 24 (ROW_GEN); kinds =
 // the zero point kind | the weights' type << 8 (ROW_GEN). shape = M (up to
-// kRowsMax) | nbc << 12 | the shift of a block's k in its chunk << 20 | the eights of the last chunk past K << 24.
+// kRowsMax) | nbc << 12 | the shift of a block's k in its chunk << 20 | the eights of the last chunk past K << 24
+// | a bias << 31.
 // The leading arguments are preloaded into SGPRs at wave launch.
 template <int BITS, int OP, bool SPLIT, int MT, int TN, int NW>
 __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
@@ -374,6 +408,24 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
       }
     }
   };
+  // The bias (its bits; zeros past N) of the columns of the tile this wavefront stores: on its way while
+  // the sums meet in LDS (fetched ahead of each store instead, an f32 bias cost f16 calls of few rows 5
+  // to 10%).
+  auto load_bias = [&](uint32_t tn) -> uint4_t {
+    uint4_t b = {0u, 0u, 0u, 0u};
+    if (!(shape >> 31)) return b;  // (types, no preloaded argument, is not waited for here)
+    const uint32_t b_dt = (types >> 16) & 0xFFu, n = (t0 + tn) * 16 + 4 * g;
+    if (b_dt == DT_F32) {
+      const auto b_rsrc = buffer_rsrc(bias, N * 4);
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) b[e] = __builtin_amdgcn_raw_buffer_load_b32(b_rsrc, (n + e) * 4, 0, 0);
+    } else {
+      const auto b_rsrc = buffer_rsrc(bias, N * 2);
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) b[e] = __builtin_amdgcn_raw_buffer_load_b16(b_rsrc, (n + e) * 2, 0, 0);
+    }
+    return b;
+  };
   if (wave < nch) {
     // Two register sets used in turn: a copy between them would wait for the loads in flight.
     Weights wa, wb;
@@ -429,6 +481,8 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
       }
     }
   }
+  uint4_t b0 = {0u, 0u, 0u, 0u};
+  if (wave < MT * TN) b0 = load_bias(wave % TN);
   __syncthreads();
   constexpr uint32_t kOwn = OP == ROW_F16 ? DT_F16 : OP == ROW_BF16 ? DT_BF16 : DT_F32;
   const bool plain = (types & 0xFFFFFFu) == (kOwn | (kOwn << 8)) && ldy % 4 == 0 &&
@@ -461,7 +515,8 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
         *reinterpret_cast<float4_t*>(static_cast<float*>(Y) + at) = v;
       }
     } else {
-      rows_store_any(v, Y, types, bias, at, n, N);
+      rows_store_any(v, Y, types, p0 == 0 ? b0 : load_bias(tn), at, n, N,
+                     ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & ((types & 0xFFu) == DT_F32 ? 15 : 7)) == 0);
     }
   }
 }

@@ -122,7 +122,8 @@ void launch_rows(const tmh_weight* w, const void* a, int a_dtype, int64_t M, int
   const uint32_t pad = static_cast<uint32_t>((w->nchunks * cw - w->K) / 4);
   const RowsArgs d{reinterpret_cast<const uint4_t*>(w->d_q), w->d_scale, static_cast<const uint8_t*>(w->d_zero), a,
                    static_cast<uint32_t>(w->nchunks), static_cast<uint32_t>(w->ntiles), static_cast<uint32_t>(lda),
-                   static_cast<uint32_t>(M) | (static_cast<uint32_t>(w->nbc) << 12) | (static_cast<uint32_t>(shift) << 20) | (pad / 2 << 24),
+                   static_cast<uint32_t>(M) | (static_cast<uint32_t>(w->nbc) << 12) | (static_cast<uint32_t>(shift) << 20) | (pad / 2 << 24) |
+                       (bias ? 1u << 31 : 0u),
                    y, ldy, static_cast<uint32_t>(w->N),
                    static_cast<uint32_t>(y_dtype) | (static_cast<uint32_t>(dot_dtype) << 8) |
                        (static_cast<uint32_t>(bias ? bias_dtype : 0) << 16) | (static_cast<uint32_t>(a_dtype) << 24),
