@@ -565,6 +565,7 @@ __device__ __forceinline__ void gemm_lds(
   constexpr int MTW = TALL ? BM / 16 : 8;
   constexpr int NTW = TALL ? 2 : 4;
   static_assert(MODE == GM_F16 || (TALL && !SPLIT), "the bf16 paths use the tall layout, one parameter per lane");
+  static_assert(MODE != GM_INT || KS == 2, "the sums grow back where the halves of a k-block meet");
   constexpr int ABUF = BM * ROWB * (splits_a(MODE) ? 2 : 1);  // LDS bytes of one A buffer (hi, then lo)
   constexpr int SES = splits_a(MODE) && WT == DT_F32 ? 4 : 2;  // bytes per stored scale
   extern __shared__ __align__(16) uint8_t lds[];
@@ -922,12 +923,6 @@ __device__ __forceinline__ void gemm_lds(
     __syncthreads();
     if (more) cur = next;
   }
-  if constexpr (MODE == GM_INT) {
-#pragma unroll
-    for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < NTW; ++nt) acc[mt][nt] *= kIntGrow<BITS>;
-  }
   if constexpr (KS == 2) {
     // The second half's partial sums through LDS (free after the k-loop's last barrier: no
     // load into it is in flight) into the first half's; the first half stores.
@@ -943,7 +938,10 @@ __device__ __forceinline__ void gemm_lds(
 #pragma unroll
       for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < NTW; ++nt) acc[mt][nt] += part[((wl * MTW + mt) * NTW + nt) * 64 + lane];
+        for (int nt = 0; nt < NTW; ++nt) {
+          acc[mt][nt] += part[((wl * MTW + mt) * NTW + nt) * 64 + lane];
+          if constexpr (MODE == GM_INT) acc[mt][nt] *= kIntGrow<BITS>;
+        }
     }
   }
   // Lane (16g + r) holds, for each (mt, nt), row mt*16 + r and the 4 columns nt*16 + 4g ...
