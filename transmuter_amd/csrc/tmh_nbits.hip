@@ -1540,14 +1540,22 @@ bool fast_path(const tmh_weight* w, const MatArgs& a) {
   return a.a_dt == TMH_F16 && w->wdtype == TMH_F16 && w->zp_kind != TMH_ZP_FLOAT;
 }
 
-// Rows of A that the LDS-tiled GEMM takes: over 64, and from 33 on (17 for vocabulary-sized N) where
-// 16-bit operands meet so many columns that its 64-row tiles fill half the CUs without a split of K
-// (those calls need no scratch memory). f16 q4 in graph replays, this GEMM against k_gemv_rows:
-// 2048->22016, M = 64 19.0 / 24.9 us (M = 24: 18 / 14.8), 1024->18000, M = 64 11.1 / 13-15,
-// 1024->151936, M = 32 35.1 / 48.7; below, 4096->12288 (768 tiles), M = 64 32.8 / 27-30.
+// Rows of A that the LDS-tiled GEMM takes: over 64, and fewer where 16-bit operands meet so many columns
+// that its 64-row tiles fill half the CUs without a split of K (those calls need no scratch memory), from
+// as many rows on as k_gemv_rows needs longer for. 1024 and 4096 tiles of 16 columns, us in graph
+// replays, this GEMM / k_gemv_rows (f16; bf16 the same within 10%):
+//  2 bits: 33 rows 1024->16400 10.2 / 15.7, 8192->16400 50 / 86; 17 rows 1024->65600 18.9 / 21.9;
+//  4 bits: 33 rows 256->16400 5.7 / 6.4, 1024-> 10.9 / 11.4, 8192-> 62.7 / 60.6, 64 rows 11.0 / 13.7 and
+//          63.5 / 80.8, blocks of 16 up to twice as far apart; 1024->65600 17 rows 21.7 / 20.2, 24 rows
+//          21.7 / 22.1, 33 rows 22.2 / 34.4; 768 tiles (4096->12288), 64 rows 32.8 / 27-30;
+//  8 bits: 1024->16400 33 rows 14.2 / 12.3, 64 rows 14.5 / 14.3, 8192->16400 33 rows 111 / 70, 64 rows
+//          111 / 88; 1024->65600 17 rows 30.0 / 20.1, 24 rows 30.5 / 22.4, 33 rows 29.9 / 34.9, 64 rows 30.5 / 41.
 bool gemm_rows(const tmh_weight* w, const MatArgs& a) {
-  return a.M > 64 || (a.M > (w->ntiles >= 4096 ? 16 : 32) && w->ntiles >= 1024 && a.a_dt == w->wdtype &&
-                      a.a_dt != TMH_F32 && a.a_vec && w->zp_kind != TMH_ZP_FLOAT);
+  if (a.M > 64) return true;
+  const bool vocabulary = w->ntiles >= 4096;
+  const int64_t least = vocabulary && w->bits == 2 ? 17 : vocabulary && w->bits == 4 ? 25 : 33;
+  return a.M >= least && w->ntiles >= (w->bits == 8 ? 4096 : 1024) && a.a_dt == w->wdtype && a.a_dt != TMH_F32 && a.a_vec &&
+         w->zp_kind != TMH_ZP_FLOAT;
 }
 
 // The operand path of the LDS-tiled prefill GEMM for a call, or -1 where it does not apply: enough
