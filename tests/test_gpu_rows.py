@@ -1,10 +1,12 @@
 """MatMulNBits of up to 64 rows in any float types (k_gemv_rows) on the GPU, at the sizes where its
-launch shapes, remainders and operand paths change, against float64 sums over the oracle's weights.
+launch shapes, remainders and operand paths change, and the calls beside it that other kernels take,
+against float64 sums over the oracle's weights.
 
 Bound per output, S = sum |a w| of its products: 2^-20 S for the f32 sums (K up to a few thousand in
 chunks of 32, each partial sum rounding by 2^-24 of its value) and the weights' own f32 rounding,
 plus half a unit in the last place of the dot's and of Y's type (2^-11 f16, 2^-8 bf16)."""
 
+import ctypes
 import zlib
 
 import numpy as np
@@ -14,6 +16,7 @@ from oracle import oracle as o
 from synth import nbits_weight
 from test_gpu_nbits import as_f64, host_float
 from transmuter_amd import PackedWeight
+from transmuter_amd._lib import BF16, F16, F32, lib
 from transmuter_amd.device import bf16_host
 from transmuter_amd.quantized import matmul_nbits
 
@@ -72,6 +75,89 @@ def test_launch_shapes(ctx, m, n, chunks, a_dtype, w_dtype):
     bias = "f32" if a_dtype == "f16" and m <= 16 else None
     y, ref, bound = check(ctx, a, a_dtype, w_dtype, k, n, 4, 32, "packed", bias, seed=n)
     assert (np.abs(y - ref) <= bound).all()
+
+
+# The shapes of several tiles or sets of rows with 2- and 8-bit weights and parameters that change within a
+# lane's group.
+@pytest.mark.parametrize("a_dtype,w_dtype", TYPES)
+@pytest.mark.parametrize("bits,block", [(2, 16), (2, 64), (4, 16), (8, 32)])
+@pytest.mark.parametrize("m,n,chunks", [(16, 4160, 9), (16, 33000, 2), (20, 5000, 3), (48, 2704, 2), (30, 16500, 2), (64, 16200, 3)])
+def test_launch_shapes_of_other_weights(ctx, m, n, chunks, bits, block, a_dtype, w_dtype):
+    k = chunks * chunk(bits) - 24
+    print(f"rows m={m} n={n} k={k} b{bits} bs{block} {a_dtype}", flush=True)
+    rng = np.random.default_rng(m * 1000 + n)
+    a = typed(rng.standard_normal((m, k)), a_dtype)
+    bias = "f32" if a_dtype == "f16" and m <= 16 else None
+    y, ref, bound = check(ctx, a, a_dtype, w_dtype, k, n, bits, block, "packed", bias, seed=n)
+    assert (np.abs(y - ref) <= bound).all()
+
+
+# 17 to 64 rows against so many columns that the prefill GEMM takes them, unsplit (from 33 rows on; against
+# 65536 columns 17 of 2 bits and 25 of 4; 8 bits from 65536 columns on), and the row counts beside.
+@pytest.mark.parametrize("a_dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("bits,block,zp", [(2, 64, "packed"), (8, 32, "none"), (8, 128, "packed"), (4, 32, "packed")])
+@pytest.mark.parametrize("m,n", [(32, 16400), (33, 16400), (64, 16384), (16, 65550), (17, 65550), (25, 65550), (33, 65550)])
+def test_few_rows_of_the_prefill_gemm(ctx, m, n, bits, block, zp, a_dtype):
+    k = 2 * chunk(bits) + 40
+    print(f"few prefill rows m={m} n={n} k={k} b{bits} bs{block} {zp} {a_dtype}", flush=True)
+    rng = np.random.default_rng(m + n)
+    a = typed(rng.standard_normal((m, k)), a_dtype)
+    y, ref, bound = check(ctx, a, a_dtype, a_dtype, k, n, bits, block, zp, None, seed=n)
+    assert (np.abs(y - ref) <= bound).all()
+
+
+CODE = {"f32": F32, "f16": F16, "bf16": BF16}
+NP = {"f32": np.float32, "f16": np.float16, "bf16": np.uint16}
+SIZE = {"f32": 4, "f16": 2, "bf16": 2}
+
+
+def check_rows(ctx, m, k, n, a_dtype, w_dtype, bits, block, zp, lda, ldy, a_off, y_off):
+    """One call over rows lda and ldy apart that start a_off and y_off values into their buffers; the rest
+    of Y's buffer stays as it was."""
+    rng = np.random.default_rng(m * 7919 + k)
+    b, s32, z = nbits_weight(rng, k, n, bits, block, zp=zp, scale_dtype=np.float32)
+    scales = typed(s32, w_dtype)
+    w = PackedWeight.upload(ctx, b, scales, z, k=k, n=n, bits=bits, block_size=block, weight_dtype=w_dtype)
+    y_dtype = a_dtype if a_dtype == w_dtype else "f32"
+    a = typed(rng.standard_normal(a_off + m * lda), a_dtype)
+    a_d, y_d = ctx.put(a), ctx.put(np.full(y_off + m * ldy + 8, 7, NP[y_dtype]))
+    a_at = ctypes.c_void_p(a_d.ptr.value + a_off * SIZE[a_dtype])
+    y_at = ctypes.c_void_p(y_d.ptr.value + y_off * SIZE[y_dtype])
+    ctx.check(lib().tmh_matmul_nbits(ctx.handle, w.handle, a_at, CODE[a_dtype], m, lda, None, 0, y_at, CODE[y_dtype], ldy, None))
+    whole = y_d.numpy()
+    w.free()
+    rows = whole[y_off:y_off + m * ldy].reshape(m, ldy)
+    assert (whole[:y_off] == 7).all() and (rows[:, n:] == 7).all() and (whole[y_off + m * ldy:] == 7).all()
+    y = as_f64(rows[:, :n], y_dtype)
+    af = as_f64(a[a_off:].reshape(m, lda)[:, :k], a_dtype)
+    dense = np.asarray(o.dequantize_weight(b, as_f64(scales, w_dtype).astype(np.float32), z, k, n, bits, block, w_dtype), np.float64)
+    ref = af @ dense.T
+    # Over 64 rows an f32 factor goes through the prefill GEMM as two bf16 parts, 16 bits and a half of it:
+    # 2^-17 for each factor and 2^-16 for the product of the low parts, left out.
+    part = 2.0 ** -15 if m > 64 and "f32" in (a_dtype, w_dtype) else 2.0 ** -20
+    bound = part * (np.abs(af) @ np.abs(dense).T) + 2 * HALF_ULP[y_dtype] * np.abs(ref) + (2.0 ** -24 if y_dtype == "f16" else 0)
+    assert (np.abs(y - ref) <= bound).all()
+
+
+PATHS = TYPES + [("f32", "f16"), ("f16", "f32"), ("bf16", "f32"), ("f16", "bf16")]
+
+
+@pytest.mark.parametrize("a_dtype,w_dtype", PATHS)
+@pytest.mark.parametrize("m,bits,block,zp", [(20, 4, 32, "packed"), (64, 4, 16, "none"), (20, 8, 64, "float"), (3, 2, 64, "packed")])
+@pytest.mark.parametrize("y_off", [0, 1, 2])
+def test_strides_and_y_off_its_alignment(ctx, m, bits, block, zp, a_dtype, w_dtype, y_off):
+    print(f"strides m={m} b{bits} bs{block} {zp} {a_dtype} {w_dtype} y_off={y_off}", flush=True)
+    check_rows(ctx, m, 264, 150, a_dtype, w_dtype, bits, block, zp, 280, 150 + (5 if y_off else 6), 0, y_off)
+
+
+# K no multiple of 8, or rows of A off 16-byte boundaries: the kernels that load value by value.
+@pytest.mark.parametrize("a_dtype,w_dtype", PATHS)
+@pytest.mark.parametrize("m", [1, 5, 17, 40, 70])
+@pytest.mark.parametrize("k,lda,a_off,bits,block,zp", [(77, 77, 0, 4, 16, "packed"), (100, 104, 0, 4, 32, "float"),
+                                                       (264, 264, 1, 8, 32, "none"), (300, 301, 2, 2, 64, "packed")])
+def test_rows_off_the_vector_loads(ctx, m, k, lda, a_off, bits, block, zp, a_dtype, w_dtype):
+    print(f"off the loads m={m} k={k} lda={lda} +{a_off} b{bits} bs{block} {zp} {a_dtype} {w_dtype}", flush=True)
+    check_rows(ctx, m, k, 75, a_dtype, w_dtype, bits, block, zp, lda, 75, a_off, 0)
 
 
 @pytest.mark.parametrize("bits,block", [(2, 16), (2, 64), (4, 16), (4, 64), (4, 256), (8, 16), (8, 32), (8, 128)])
