@@ -354,7 +354,6 @@ __device__ __forceinline__ void moe_gemm_f16(
   constexpr int PIECES = ROWS * PPR;             // per chunk
   constexpr int DMA = (PIECES + 511) / 512;      // load instructions of a wavefront per chunk of A
   constexpr int NW = EPI == EPI_GLU ? 2 : 1;
-  constexpr int STEP_LOADS = DMA + NW * (1 + NJ * (HAS_ZP ? 2 : 1));  // of a wavefront per step
   constexpr int AHEAD = moe_ahead(EPI, MT);
   constexpr uint32_t STAGES = AHEAD + 1;
   extern __shared__ __align__(16) uint8_t lds[];  // STAGES chunks of the item's rows of A
@@ -469,33 +468,46 @@ __device__ __forceinline__ void moe_gemm_f16(
     constexpr int MA = decltype(ma)::value;
     WStage w0, w1, w2;
     const uint32_t total = static_cast<uint32_t>(ng) * nch;
-    uint32_t cl = 0, sl = 0, stage_l = 0;  // chunk, step and stage of the next loads
+    uint32_t cl = 0;  // chunk and group of the next loads
     int gl = 0;
-    auto load_next = [&](WStage& st) {
-      load_a(cl, stage_l, sl < total);
-      load_w(gl, cl, sl < total, st);
-      ++sl;
-      stage_l = stage_l + 1 == STAGES ? 0 : stage_l + 1;
+    // A step's rows first, then its weights: two ahead, every weight load's address goes through the asm
+    // between them, so none is issued ahead of the rows, and loads return in the order of their issue.
+    auto load_next = [&](WStage& st, uint32_t stage, bool real) {
+      load_a(cl, stage, real);
+      uint32_t c_w = cl;
+      if constexpr (AHEAD == 2) {
+        c_w = __builtin_amdgcn_readfirstlane(cl);
+        asm volatile("" : "+s"(c_w) : : "memory");
+      }
+      load_w(gl, c_w, real, st);
       if (++cl == nch) {
         cl = 0;
         ++gl;
       }
     };
-    uint32_t c = 0, stage = 0;
+    // Two ahead: waits for a step's weights, and so for this wavefront's rows of that step, loaded ahead
+    // of them: the asm reads the weights, and the compiler counts the wait for them itself, wherever it
+    // put the loads of the later steps, which stay in flight. (A count by hand over weights and rows
+    // holds only as long as the compiler leaves every weight load on its side of the barrier.)
+    auto arrived = [&](const WStage& st) {
+#pragma unroll
+      for (int v = 0; v < NW; ++v)
+        if constexpr (AHEAD == 2) asm volatile("" : : "v"(st.w[v]) : "memory");
+    };
+    uint32_t c = 0;
     int gi = 0;
-    auto step = [&](const WStage& cur, WStage& far) {
-      // The loads of step s + 1 may stay in flight. (The count holds as long as none of them is moved past
-      // the barrier, which the compiler may do with the weights' ones: over all paths of every build's
-      // assembly no row load older than step s + 1 is in flight at a barrier. Look again when this changes.)
-      constexpr int kWait = (AHEAD - 1) * STEP_LOADS;
-      __builtin_amdgcn_s_waitcnt((kWait & 15) | (7 << 4) | ((kWait >> 4) << 14));
+    // Step s, whose rows lie in stage s % STAGES: a constant, as the loop below turns once per ring.
+    auto step = [&](auto stage_c, uint32_t s, const WStage& cur, const WStage& next, WStage& far) {
+      constexpr uint32_t STAGE = decltype(stage_c)::value;
+      // The last step's LDS reads are done (its stage is filled next) and, one ahead, so is every load.
+      __builtin_amdgcn_s_waitcnt(AHEAD == 2 ? 15 | (7 << 4) | (3 << 14) : 7 << 4);
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-      load_next(far);
+      load_next(far, (STAGE + AHEAD) % STAGES, s + AHEAD < total);
       __builtin_amdgcn_sched_barrier(0);
-      const uint8_t* abase = lds + stage * (ROWS * ROWB);
+      const uint8_t* abase = lds + STAGE * (ROWS * ROWB);
 #pragma unroll
       for (int i = 0; i < STEPS; ++i) {
         const int piece = g * (GW / 8) + i;
@@ -514,7 +526,6 @@ __device__ __forceinline__ void moe_gemm_f16(
             acc[v][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, af[mt], acc[v][mt], 0, 0, 0);
         }
       }
-      stage = stage + 1 == STAGES ? 0 : stage + 1;
       if (++c == nch) {
         if (active_g(gi)) store_group(gi);
 #pragma unroll
@@ -524,16 +535,20 @@ __device__ __forceinline__ void moe_gemm_f16(
         c = 0;
         ++gi;
       }
+      arrived(next);
     };
-    load_next(w0);
-    if constexpr (AHEAD == 2) load_next(w1);
+    load_next(w0, 0, true);
+    __builtin_amdgcn_sched_barrier(0);  // (mixed with the next step's, the first wait would take both)
+    if constexpr (AHEAD == 2) load_next(w1, 1, total > 1);
+    __builtin_amdgcn_sched_barrier(0);
+    arrived(w0);
     for (uint32_t s = 0;;) {
-      step(w0, AHEAD == 2 ? w2 : w1);
+      step(std::integral_constant<uint32_t, 0>{}, s, w0, w1, AHEAD == 2 ? w2 : w1);
       if (++s == total) break;
-      step(w1, w0);
+      step(std::integral_constant<uint32_t, 1>{}, s, w1, AHEAD == 2 ? w2 : w0, w0);
       if (++s == total) break;
       if constexpr (AHEAD == 2) {
-        step(w2, w1);
+        step(std::integral_constant<uint32_t, 2>{}, s, w2, w0, w1);
         if (++s == total) break;
       }
     }
