@@ -153,3 +153,34 @@ def test_gather_and_qmoe_stamping_builds(ctx):
     tl.free()
     for w in ws:
         w.free()
+
+
+def test_qmoe_of_few_rows_stamps_its_products(ctx):
+    """Few rows an expert take k_moe_rows: its launches are recorded too (a recorded call routes and plans
+    in two launches), and compute the same bits."""
+    from transmuter_amd.moe import ExpertWeight
+
+    rng = np.random.default_rng(7)
+    e, kk, h, inter, t = 16, 2, 256, 96, 9
+    ws = []
+    for n_, k_ in ((inter, h), (inter, h), (h, inter)):
+        packed = rng.integers(0, 256, (e, n_, k_ // 2), dtype=np.uint8)
+        scales = (np.abs(rng.standard_normal((e, n_, k_ // 32))) * 0.01 + 1e-4).astype(np.float16)
+        ws.append(ExpertWeight.upload(ctx, packed, scales, None, bits=4, block_size=32, dtype="f16"))
+    x = ctx.put(rng.standard_normal((t, h)).astype(np.float16))
+    router = ctx.put(rng.standard_normal((t, e)).astype(np.float32))
+    ys = [ctx.empty((t, h), "f16") for _ in range(2)]
+    tl = Timeline(ctx, 1 << 16)
+    for i, yy in enumerate(ys):
+        if i == 1:
+            tl.begin()
+        ctx.check(lib().tmh_qmoe(ctx.handle, x.ptr, F16, t, h, router.ptr, F32, e, kk, ws[0].handle, None,
+                                 ws[2].handle, None, ws[1].handle, None, F16, 4, 0, 1.0, 0.0, 0.0, yy.ptr, None))
+    tl.end()
+    ctx.synchronize()
+    print("timeline qmoe, few rows", flush=True)
+    assert np.array_equal(ys[0].numpy().view(np.uint16), ys[1].numpy().view(np.uint16))
+    _check_launches(tl, ["k_moe_route", "k_moe_plan", "k_moe_rows", "k_moe_rows", "k_moe_combine"])
+    tl.free()
+    for w in ws:
+        w.free()

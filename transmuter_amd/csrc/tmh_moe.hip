@@ -608,8 +608,9 @@ __global__ __launch_bounds__(512) void k_moe_gemm_f16_tl(
 // then by the instructions that unpack (zero points known to be absent take a fifth of them away).
 // 2048/768 q4, graphless calls: one token, top 8 of 128 experts 41.4 -> 21.5 us, 8 tokens 58.6 -> 47.6
 // (fc1 and fc3 27.8 -> 23.9 us traced, fc2 17.2 -> 12.5).
+// (The body; k_moe_rows and its stamping build k_moe_rows_tl below are the kernels.)
 template <int BITS, bool HAS_ZP, bool SPLIT, int EPI, int TN, int NW>
-__global__ __launch_bounds__(64 * NW) void k_moe_rows(
+__device__ __forceinline__ void moe_rows(
     const uint4_t* __restrict__ qt, const uint16_t* __restrict__ sc, const uint8_t* __restrict__ zp,
     const uint4_t* __restrict__ qt2, const uint16_t* __restrict__ sc2, const uint8_t* __restrict__ zp2, int tile_off2,
     int ntiles, int nchunks, int nbc, int bsc_shift, int tiles_per_expert, int out_tiles,
@@ -769,6 +770,36 @@ __global__ __launch_bounds__(64 * NW) void k_moe_rows(
     *reinterpret_cast<uint2*>(out + static_cast<int64_t>(orow) * ldo + n) =
         make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
   }
+}
+
+template <int BITS, bool HAS_ZP, bool SPLIT, int EPI, int TN, int NW>
+__global__ __launch_bounds__(64 * NW) void k_moe_rows(
+    const uint4_t* __restrict__ qt, const uint16_t* __restrict__ sc, const uint8_t* __restrict__ zp,
+    const uint4_t* __restrict__ qt2, const uint16_t* __restrict__ sc2, const uint8_t* __restrict__ zp2, int tile_off2,
+    int ntiles, int nchunks, int nbc, int bsc_shift, int tiles_per_expert, int out_tiles,
+    const _Float16* __restrict__ A, int a_rows, int lda, const int* __restrict__ perm, int perm_div,
+    const int4* __restrict__ items, const int* __restrict__ n_items, const void* __restrict__ bias1,
+    const void* __restrict__ bias2, int bias_dt, int bias_ld, int act, float alpha, float beta, float limit,
+    _Float16* __restrict__ out, int ldo, const int* __restrict__ out_perm) {
+  moe_rows<BITS, HAS_ZP, SPLIT, EPI, TN, NW>(
+      qt, sc, zp, qt2, sc2, zp2, tile_off2, ntiles, nchunks, nbc, bsc_shift, tiles_per_expert, out_tiles, A, a_rows, lda,
+      perm, perm_div, items, n_items, bias1, bias2, bias_dt, bias_ld, act, alpha, beta, limit, out, ldo, out_perm);
+}
+
+template <int BITS, bool HAS_ZP, bool SPLIT, int EPI, int TN, int NW>
+__global__ __launch_bounds__(64 * NW) void k_moe_rows_tl(
+    const uint4_t* __restrict__ qt, const uint16_t* __restrict__ sc, const uint8_t* __restrict__ zp,
+    const uint4_t* __restrict__ qt2, const uint16_t* __restrict__ sc2, const uint8_t* __restrict__ zp2, int tile_off2,
+    int ntiles, int nchunks, int nbc, int bsc_shift, int tiles_per_expert, int out_tiles,
+    const _Float16* __restrict__ A, int a_rows, int lda, const int* __restrict__ perm, int perm_div,
+    const int4* __restrict__ items, const int* __restrict__ n_items, const void* __restrict__ bias1,
+    const void* __restrict__ bias2, int bias_dt, int bias_ld, int act, float alpha, float beta, float limit,
+    _Float16* __restrict__ out, int ldo, const int* __restrict__ out_perm, uint32_t* __restrict__ tl) {
+  const TlStart t0 = tl_clock();
+  moe_rows<BITS, HAS_ZP, SPLIT, EPI, TN, NW>(
+      qt, sc, zp, qt2, sc2, zp2, tile_off2, ntiles, nchunks, nbc, bsc_shift, tiles_per_expert, out_tiles, A, a_rows, lda,
+      perm, perm_div, items, n_items, bias1, bias2, bias_dt, bias_ld, act, alpha, beta, limit, out, ldo, out_perm);
+  tl_stamp(tl, t0);
 }
 
 // The same product for any float types (A in a_dt, weights dequantized in WDT, out in out_dt):
@@ -1049,13 +1080,18 @@ void go_moe_rows(const tmh_weight* w, int tpe, const void* A, int a_rows, int ld
                  hipStream_t s) {
   const tmh_weight* w2 = ep.w2 ? ep.w2 : w;
   const dim3 grid(static_cast<unsigned>((ep.out_tiles + TN - 1) / TN), static_cast<unsigned>(work.max_items));
-  k_moe_rows<BITS, HAS_ZP, SPLIT, EPI, TN, NW><<<grid, 64 * NW, 0, s>>>(
-      reinterpret_cast<const uint4_t*>(w->d_q), static_cast<const uint16_t*>(w->d_scale),
-      static_cast<const uint8_t*>(w->d_zero), reinterpret_cast<const uint4_t*>(w2->d_q),
-      static_cast<const uint16_t*>(w2->d_scale), static_cast<const uint8_t*>(w2->d_zero), ep.tile_off2,
-      static_cast<int>(w->ntiles), static_cast<int>(w->nchunks), w->nbc, bsc_shift_moe(w), tpe, ep.out_tiles,
-      static_cast<const _Float16*>(A), a_rows, lda, perm, perm_div, work.items, work.n_items, ep.bias1, ep.bias2, ep.bias_dt,
-      ep.bias_ld, ep.act, ep.alpha, ep.beta, ep.limit, static_cast<_Float16*>(out), ldo, ep.out_perm);
+#define TMH_MOE_ARGS                                                                                                  \
+  reinterpret_cast<const uint4_t*>(w->d_q), static_cast<const uint16_t*>(w->d_scale),                                 \
+      static_cast<const uint8_t*>(w->d_zero), reinterpret_cast<const uint4_t*>(w2->d_q),                              \
+      static_cast<const uint16_t*>(w2->d_scale), static_cast<const uint8_t*>(w2->d_zero), ep.tile_off2,               \
+      static_cast<int>(w->ntiles), static_cast<int>(w->nchunks), w->nbc, bsc_shift_moe(w), tpe, ep.out_tiles,         \
+      static_cast<const _Float16*>(A), a_rows, lda, perm, perm_div, work.items, work.n_items, ep.bias1, ep.bias2,     \
+      ep.bias_dt, ep.bias_ld, ep.act, ep.alpha, ep.beta, ep.limit, static_cast<_Float16*>(out), ldo, ep.out_perm
+  if (uint32_t* tl = timeline_slots(TMH_TL_MOE_ROWS, static_cast<int64_t>(grid.x) * grid.y * NW))
+    k_moe_rows_tl<BITS, HAS_ZP, SPLIT, EPI, TN, NW><<<grid, 64 * NW, 0, s>>>(TMH_MOE_ARGS, tl);
+  else
+    k_moe_rows<BITS, HAS_ZP, SPLIT, EPI, TN, NW><<<grid, 64 * NW, 0, s>>>(TMH_MOE_ARGS);
+#undef TMH_MOE_ARGS
 }
 
 template <int BITS, bool HAS_ZP, bool SPLIT, int EPI>
