@@ -18,13 +18,13 @@
 //  ROW_F16   f16 A and weights: exact f16 weights (q - zero) * scale (unpack_step);
 //  ROW_BF16  bf16 A and weights: (q - zero) * scale formed in f32 and rounded once to bf16, as the
 //            reference's bf16 dequantization rounds it (a scale of 2^117 and more overflows on the way,
-//            natural_values: rows_exact forms the sums of such weights);
+//            natural_values: rows_again forms the sums of such weights);
 //  ROW_INT   f32 A and f32 weights of blocks of 32 and more: q - zero is a whole number of at most
 //            8 bits and so exact in bf16, a value of A is the exact sum of three bf16 parts, and a
 //            step's 32 products sit in one block, whose f32 scale multiplies the step's f32 sums:
 //            three MFMAs and four FMAs a lane per step, with f32 products throughout. (A step's sum
 //            before its scale can pass f32's range, from |a| near 4e34 with 8 bits and 7e35 with 4
-//            on: it comes out infinite or NaN then, and rows_exact forms the sums again.);
+//            on: it comes out infinite or NaN then, and rows_again forms the sums again.);
 //  ROW_GEN   every other combination (mixed types, float zero points, f32 weights in blocks of 16 or
 //            of 2 bits): the weights dequantize in f32 as the reference does in their type, and
 //            three bf16 parts of each factor (exact) meet in all nine products, so that none is
@@ -47,7 +47,7 @@ typedef __bf16 rows_bf16x8_t __attribute__((ext_vector_type(8)));
 // Eight f32 values as the sum of three bf16 parts each: the top 8 bits of the significand, the next
 // 8 and the last 8 (cut, not rounded: every part is exact, and no part of a finite value
 // overflows; below 2^-110 the last bits fall under bf16's own range). An infinity leaves a NaN
-// behind: the sums it enters are formed again (rows_exact).
+// behind: the sums it enters are formed again (rows_again).
 __device__ __forceinline__ void split3(const float (&a)[8], uint4_t (&part)[3]) {
   float rest[8];
   uint32_t top[8];
@@ -122,48 +122,115 @@ __device__ __noinline__ void rows_store_any(float4_t v, void* Y, uint32_t types,
   }
 }
 
-// One wavefront's sums of four consecutive columns of one row again, one f32 FMA per product as
-// k_matmul_general forms them, over its chunks c0, c0 + step, ...: for the sums that came out infinite or
-// NaN, where the parts of a factor may be at fault (0 times an infinity's other part, a weight whose
-// scale lies at the end of its type). Rare, so nothing here is made fast, and out of line: inside the
-// kernel its code spread the rest apart (bf16 M = 8 1024 -> 4096 3.52 us inside, 3.45 here, 3.36 without it).
+// (q - z) * s of eight values as the reference dequantizes them in the weights' type: one uniform branch
+// over the type, not two a value.
+__device__ __forceinline__ void dequantize8(float (&q)[8], float z, float s, int w_dt) {
+  if (w_dt == DT_F32) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[e] = (q[e] - z) * s;
+  } else if (w_dt == DT_F16) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[e] = round_to<DT_F16>(round_to<DT_F16>(q[e] - z) * s);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[e] = round_to<DT_BF16>(round_to<DT_BF16>(q[e] - z) * s);
+  }
+}
+
+// Four consecutive columns' sums v of one row, over the chunks c0, c0 + step, ..., with those that are
+// infinite or NaN formed again, one f32 FMA per product as k_matmul_general forms them: where the parts
+// of a factor may be at fault (0 times an infinity's other part, a block's sum past f32's range ahead of
+// its scale, a weight whose scale lies at the end of its type). Not where A's row holds a NaN, which no
+// other sum would change, nor (scales_only) where no scale is that large. Out of line: inside the kernel
+// its code spread the rest apart (bf16 M = 8 1024 -> 4096 3.52 us, 3.45 out of line). us of a call whose A
+// holds a NaN / an infinity / neither: f32 M = 16 1024 -> 4096 6.2 / 31.9 / 5.1 (k_matmul_general 55), bf16
+// M = 8 6.7 / 6.7 / 3.4.
 template <int BITS>
-__device__ __noinline__ float4_t rows_exact(const uint4_t* qt, const void* sc, const uint8_t* zp, const void* A, int a_dt,
-                                               int w_dt, uint32_t zk, uint32_t tile, uint32_t col, uint32_t a_at,
-                                               uint32_t nch, uint32_t nbc, uint32_t bsc_shift, uint32_t K, uint32_t c0,
-                                               uint32_t step) {
-  constexpr uint32_t CW = 512 / BITS, GW = CW / 4;
+__device__ __noinline__ float4_t rows_again(float4_t v, const uint4_t* qt, const void* sc, const uint8_t* zp, const void* A,
+                                            int a_dt, int w_dt, uint32_t zk, uint32_t tile, uint32_t col, uint32_t a_at,
+                                            uint32_t nch, uint32_t nbc, uint32_t bsc_shift, uint32_t K, uint32_t c0,
+                                            uint32_t step, bool scales_only) {
+  constexpr uint32_t CW = 512 / BITS, GW = CW / 4, STEPS = GW / 8;
+  if (v[0] * 0.f + v[1] * 0.f + v[2] * 0.f + v[3] * 0.f == 0.f) return v;
+  if (scales_only) {
+    uint32_t most = 0;  // the largest bf16 scale's magnitude, in the upper half
+    for (uint32_t c = c0; c < nch; c += step)
+#pragma unroll 2
+      for (uint32_t b = 0; b < nbc; ++b) {
+        const uint2 s4 = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(sc) + ((tile * nch + c) * nbc + b) * 16 + col);
+        most = max(max(most, max((s4.x << 16) & 0x7FFF0000u, s4.x & 0x7FFF0000u)),
+                   max((s4.y << 16) & 0x7FFF0000u, s4.y & 0x7FFF0000u));
+      }
+    const bool large = most >= 0x7A000000u;  // 2^117
+    if (!large) return v;
+  }
+  // Eight values of A from k on: 16-byte loads, as gemv_rows_ok has A aligned and K a multiple of 8.
+  auto load8 = [&](uint32_t k, float (&a)[8]) {
+    if (a_dt == DT_F32) {
+      const auto* p = reinterpret_cast<const float4_t*>(static_cast<const float*>(A) + a_at + k);
+      const float4_t x = p[0], y = p[1];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        a[j] = x[j];
+        a[4 + j] = y[j];
+      }
+    } else {
+      const uint4_t x = *reinterpret_cast<const uint4_t*>(static_cast<const uint16_t*>(A) + a_at + k);
+      const uint32_t h[4] = {x[0], x[1], x[2], x[3]};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const auto u = static_cast<uint16_t>(h[j / 2] >> (16 * (j % 2)));
+        a[j] = a_dt == DT_F16 ? f16_bits_to_f32(u) : bf16_bits_to_f32(u);
+      }
+    }
+  };
+  bool nan = false;
+#pragma unroll 1
+  for (uint32_t c = c0; c < nch; c += step) {
+    const uint32_t end = min(c * CW + CW, K);
+#pragma unroll 2
+    for (uint32_t k = c * CW; k < end; k += 8) {
+      float a[8];
+      load8(k, a);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) nan |= a[j] != a[j];
+    }
+  }
+  if (nan) return v;
   float4_t sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
   for (uint32_t c = c0; c < nch; c += step)
 #pragma unroll 1
-    for (uint32_t kg = 0; kg < 4; ++kg)
+    for (uint32_t kge = 0; kge < 16; ++kge) {  // a k-group of a column: its parameters' loads in one go
+      const uint32_t kg = kge >> 2, e = kge & 3, k0 = c * CW + kg * GW;
+      const uint4_t w = qt[(tile * nch + c) * 64 + kg * 16 + col + e];
+      float s[STEPS], z[STEPS], x = 0.f;
 #pragma unroll
-      for (uint32_t i = 0; i < GW / 8; ++i) {
-        const uint32_t kc = kg * GW + 8 * i, k = c * CW + kc;
-        if (k >= K) break;  // K is a multiple of 8
-        float a[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) a[j] = load_float_rt(A, a_dt, a_at + k + j);
-#pragma unroll 1
-        for (uint32_t e = 0; e < 4; ++e) {
-          const uint32_t at = ((tile * nch + c) * nbc + (kc >> bsc_shift)) * 16 + col + e;
-          const float s = load_float_rt(sc, w_dt, at);
-          const float z = zk == TMH_ZP_FLOAT ? reinterpret_cast<const float*>(zp)[at]
-                          : zk == TMH_ZP_PACKED
-                              ? static_cast<float>(zp_field<BITS>(zp[zp_byte<BITS>(at)], zp_shift<BITS>(static_cast<int>(col + e))))
-                              : static_cast<float>(1 << (BITS - 1));
-          float q[8], x = 0.f;
-          natural_values<BITS>(qt[(tile * nch + c) * 64 + kg * 16 + col + e], static_cast<int>(i), 1.f, 0.f, q);
-#pragma unroll
-          for (int f = 0; f < 4; ++f) x = f == static_cast<int>(e) ? sum[f] : x;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) x = fmaf(round_rt(round_rt(q[j] - z, w_dt) * s, w_dt), a[j], x);
-#pragma unroll
-          for (int f = 0; f < 4; ++f) sum[f] = f == static_cast<int>(e) ? x : sum[f];
-        }
+      for (uint32_t i = 0; i < STEPS; ++i) {
+        const uint32_t at = ((tile * nch + c) * nbc + ((kg * GW + 8 * i) >> bsc_shift)) * 16 + col + e;
+        s[i] = load_float_rt(sc, w_dt, at);
+        z[i] = zk == TMH_ZP_FLOAT ? reinterpret_cast<const float*>(zp)[at]
+               : zk == TMH_ZP_PACKED ? static_cast<float>(zp_field<BITS>(zp[zp_byte<BITS>(at)], zp_shift<BITS>(col + e)))
+                                     : static_cast<float>(1 << (BITS - 1));
       }
-  return sum;
+#pragma unroll
+      for (int f = 0; f < 4; ++f) x = f == static_cast<int>(e) ? sum[f] : x;
+#pragma unroll
+      for (uint32_t i = 0; i < STEPS; ++i) {
+        if (k0 + 8 * i >= K) break;
+        float a[8], q[8];
+        load8(k0 + 8 * i, a);
+        natural_values<BITS>(w, static_cast<int>(i), 1.f, 0.f, q);
+        dequantize8(q, z[i], s[i], w_dt);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x = fmaf(q[j], a[j], x);
+      }
+#pragma unroll
+      for (int f = 0; f < 4; ++f) sum[f] = f == static_cast<int>(e) ? x : sum[f];
+    }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = v[e] * 0.f == 0.f ? v[e] : sum[e];
+  return v;
 }
 
 // types = the type of Y | the dot's << 8 | the bias's << 16 (0: none) | A's << 24 (ROW_GEN); kinds =
@@ -377,17 +444,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
           const float z = zk == TMH_ZP_FLOAT ? __builtin_bit_cast(float, zraw) : static_cast<float>(zero_of(zraw));
           float q[8];
           natural_values<BITS>(st.w[tn], i, 1.f, 0.f, q);  // q itself: a float zero point is subtracted as it is
-          // (One uniform branch over the type a step, not two a value.)
-          if (w_dt == DT_F32) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) q[e] = (q[e] - z) * s;
-          } else if (w_dt == DT_F16) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) q[e] = round_to<DT_F16>(round_to<DT_F16>(q[e] - z) * s);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) q[e] = round_to<DT_BF16>(round_to<DT_BF16>(q[e] - z) * s);
-          }
+          dequantize8(q, z, s, w_dt);
           uint4_t wp[3];
           split3(q, wp);
 #pragma unroll
@@ -457,7 +514,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) rows_red[(wave * MT * TN + mt * TN + tn) * 64 + lane] = acc[mt][tn];
-  if constexpr (OP != ROW_F16) {
+  if constexpr (OP == ROW_INT || OP == ROW_GEN) {
     float odd = 0.f;  // NaN where a sum is infinite or NaN, else 0
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -470,14 +527,9 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
       for (int p = 0; p < MT * TN; ++p) {
         const uint32_t m = m0 + p / TN * 16 + r, tile = t0 + p % TN;
         float4_t* const mine = rows_red + (wave * MT * TN + p) * 64 + lane;
-        const float4_t v = *mine;
-        if (m >= M || tile >= ntiles || v[0] * 0.f + v[1] * 0.f + v[2] * 0.f + v[3] * 0.f == 0.f) continue;
-        const float4_t x = rows_exact<BITS>(qt, sc, zp, A, types >> 24, (kinds >> 8) & 0xFFu, kinds & 0xFFu, tile, 4 * g,
-                                            m * lda, nch, nbc, bsc_shift, K, wave, NW);
-        float4_t out;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) out[e] = v[e] * 0.f == 0.f ? v[e] : x[e];
-        *mine = out;
+        if (m < M && tile < ntiles)
+          *mine = rows_again<BITS>(*mine, qt, sc, zp, A, types >> 24, (kinds >> 8) & 0xFFu, kinds & 0xFFu, tile, 4 * g, m * lda,
+                                   nch, nbc, bsc_shift, K, wave, NW, false);
       }
     }
   }
@@ -517,6 +569,14 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_rows(
     } else {
       rows_store_any(v, Y, types, p0 == 0 ? b0 : load_bias(tn), at, n, N,
                      ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & ((types & 0xFFu) == DT_F32 ? 15 : 7)) == 0);
+    }
+    // bf16 weights fail at the largest scales alone: looked for behind the store, over all of K (ahead of
+    // the sums' meeting the search cost every bf16 call up to 2.5%).
+    if constexpr (OP == ROW_BF16) {
+      if (__builtin_expect(v[0] * 0.f + v[1] * 0.f + v[2] * 0.f + v[3] * 0.f != 0.f, 0))
+        rows_store_any(rows_again<BITS>(v, qt, sc, zp, A, DT_BF16, DT_BF16, kinds & 0xFFu, t0 + tn, 4 * g, m * lda, nch, nbc,
+                                        bsc_shift, K, 0, 1, true),
+                       Y, types, p0 == 0 ? b0 : load_bias(tn), at, n, N, false);
     }
   }
 }
