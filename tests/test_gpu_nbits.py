@@ -160,8 +160,9 @@ MATMUL_CASES = [
     (8, 64, "none", 1024, 520, [100, 300], "bf16", "bf16", None),
     (4, 32, "packed", 200, 40, [70], "bf16", "bf16", None),
     (2, 64, "packed", 512, 96, [100], "bf16", "bf16", None),
-    # the split path (A and weights as bf16 hi + lo, three MFMAs): f32 A and weights, mixed types,
-    # float zero points, 2- and 8-bit, K off a chunk, ragged M and N
+    # the paths with a split A: f32 A and weights (whole-number weights, A as bf16 hi + lo, two MFMAs),
+    # and mixed types, float zero points and 2 bits (weights as hi + lo too, three); 8-bit, K off a
+    # chunk, ragged M and N
     (4, 128, "packed", 2048, 2048, [256, 300], "f32", "f32", None),
     (4, 32, "none", 200, 40, [70, 129], "f32", "f32", "f32"),
     (4, 32, "float", 1024, 520, [100, 300], "f16", "f16", None),

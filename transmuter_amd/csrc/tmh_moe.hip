@@ -1317,9 +1317,8 @@ int tmh_qmoe(tmh_ctx* ctx, const void* d_x, int x_dtype, int64_t T, int64_t H, c
   if (k <= 0 || k > 32 || k > E) return fail(ctx, TMH_ERR_UNSUPPORTED, "QMoE k must be in 1..min(32, experts), got %d", k);
   if (activation < ACT_RELU || activation > ACT_SWIGLU) return fail(ctx, TMH_ERR_UNSUPPORTED, "QMoE activation %d", activation);
   if (T < 0 || H <= 0) return fail(ctx, TMH_ERR_INVALID, "QMoE sizes must be positive");
-  // Work items are numbered expert << 16 | item, with at least kMoeRows rows per item, and an
-  // expert receives at most one row per token (the k experts of a token are distinct): T tokens
-  // must not give an expert more than 2^16 items.
+  // (An expert receives at most one row per token, the k experts of a token being distinct: no expert
+  // has more than 2^16 items of kMoeRows rows. The bound is part of the entry point, not of the items.)
   if ((T + kMoeRows - 1) / kMoeRows > (int64_t(1) << 16))
     return fail(ctx, TMH_ERR_UNSUPPORTED, "QMoE supports at most %lld tokens per call, got %lld",
                 (long long)kMoeRows << 16, (long long)T);

@@ -393,9 +393,10 @@ constexpr int kGemmBM = 256;  // largest tile height: bounds the A rows a launch
 //           (the hi and lo rows of A) and four FMAs a lane, in place of three MFMAs and the splitting
 //           of every weight, and no rounding of the weights. They enter as (q - zero) times 2^-9 (4
 //           bits) or 2^-13 (8 bits), exact too, so that no block's sum passes A's own range before its
-//           scale, and the sums take the power back at the end: full precision down to outputs of 1e-35. 509 x 1024 -> 6144 (kernel alone, traced):
-//           32.3 -> 27.3 us; the four projections of a layer of that width, with the splitting of A and
-//           the split-K sums, 121.6 -> 97.5 us; relative error against float64 4.5e-6 -> 2.5e-6.
+//           scale, and the sums take the power back at the end (under scales up to 1, outputs keep their
+//           precision down to 1e-34). 509 x 1024 -> 6144 (kernel alone, traced): 32.3 -> 27.3 us; the four
+//           projections of a layer of that width, with the splitting of A and the split-K sums, 121.6 ->
+//           97.5 us; relative error against float64 4.5e-6 -> 2.5e-6.
 enum : int { GM_F16 = 0, GM_BF16 = 1, GM_SPLIT = 2, GM_INT = 3 };
 // What GM_INT's sums are multiplied by at the end: above 32 times the largest |q - zero|.
 template <int BITS>
@@ -529,7 +530,7 @@ __device__ __noinline__ void store_quad_any(float4_t v, void* Y, int y_dt, int d
 // (The body; k_gemm_lds and its stamping build k_gemm_lds_tl below are the kernels.)
 // MODE (GM_*) and WT (GM_SPLIT: the weights' type) select the operand path; zk is the zero
 // point kind (TMH_ZP_*) read by GM_SPLIT, whose zero points are packed (BITS bits per parameter
-// entry) or f32 (float) per entry. For GM_SPLIT, A is the bf16 hi rows [M][lda] followed by the lo rows.
+// entry) or f32 (float) per entry. Where A is split, it is the bf16 hi rows [M][lda] followed by the lo rows.
 template <int BITS, bool HAS_ZP, bool SPLIT, int WN, int BM, int KS, bool TL, int MODE, int WT>
 __device__ __forceinline__ void gemm_lds(
     const uint4_t* __restrict__ qt, const void* __restrict__ sc, const void* __restrict__ zp,
@@ -1106,7 +1107,7 @@ __global__ __launch_bounds__(128 * WN * KS) void k_gemm_lds_tl(
                                                             chunks_per_split, ws, zk, tl);
 }
 
-// GM_SPLIT's A operand: A [M, K] of type ADT (rows lda apart) as bf16 hi = bf16(a) and lo =
+// The split A operand of GM_SPLIT and GM_INT: A [M, K] of type ADT (rows lda apart) as bf16 hi = bf16(a) and lo =
 // bf16(a - hi) (a - hi is exact in f32), each [M, Kp] with the rows zero-padded from K to Kp
 // (whole chunks), the lo rows after all the hi rows. One thread per 8 consecutive values of a row.
 template <int ADT>
@@ -1316,9 +1317,9 @@ struct MatArgs {
   int y_dt, dot_dt;
   int64_t ldy;
   float* ws = nullptr;       // split-K partial sums (gemm_scratch), resolved by the entry point
-  void* a_split = nullptr;   // GM_SPLIT's hi and lo rows of A (gemm_scratch)
+  void* a_split = nullptr;   // split A: its hi and lo rows (gemm_scratch)
   size_t split_cap = SIZE_MAX;  // most bytes of partial sums the plan may use
-  bool no_split_a = false;   // no scratch memory for GM_SPLIT's rows of A: the general kernel runs
+  bool no_split_a = false;   // no scratch memory for split rows of A: k_gemv_rows runs (k_matmul_general where it does not apply)
 };
 
 int bsc_shift_of(const tmh_weight* w) {
@@ -1458,7 +1459,7 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t ntiles, int64_t nchunks, int bi
   return best;
 }
 
-// A operand of one GEMM launch: the caller's A, or GM_SPLIT's hi/lo rows (K padded to whole chunks).
+// A operand of one GEMM launch: the caller's A, or its hi/lo rows (K padded to whole chunks).
 struct GemmA {
   const void* a;
   int64_t K, lda;
@@ -1584,7 +1585,7 @@ int gemm_mode(const tmh_weight* w, const MatArgs& a) {
 // Most bytes of partial sums a call's plan may keep: none up to 64 rows (see gemm_rows).
 size_t split_cap_of(const MatArgs& a) { return a.M > 64 ? a.split_cap : 0; }
 
-// Scratch memory of one call: GM_SPLIT's hi and lo rows of A, then the f32 partial sums of a plan
+// Scratch memory of one call: a split A's hi and lo rows, then the f32 partial sums of a plan
 // that splits K (splits * M * N), each 256-byte aligned; zeros where the call needs none.
 struct GemmScratch {
   size_t a_split = 0, partials = 0;
@@ -1629,7 +1630,7 @@ void launch_fast_bits(const tmh_weight* w, const MatArgs& a, hipStream_t s) {
   else launch_fast_variant<BITS, false, false>(w, a, s);
 }
 
-// The prefill GEMM on operand path `mode` (gemm_mode), with GM_SPLIT's hi/lo rows of A made first.
+// The prefill GEMM on operand path `mode` (gemm_mode), with the hi/lo rows of a split A made first.
 template <int BITS>
 void launch_gemm_bits(tmh_ctx* ctx, const tmh_weight* w, const MatArgs& a, hipStream_t s, int mode) {
   const GemmPlan p = plan_gemm(a.M, w->N, w->ntiles, w->nchunks, BITS, cus_of(ctx), split_cap_of(a), mode);
@@ -2328,9 +2329,10 @@ int tmh_matmul_nbits_noalloc(tmh_ctx* ctx, const tmh_weight* w, const void* d_a,
   bool run = false;
   TMH_TRY(prepare_matmul(ctx, w, d_a, a_dtype, M, lda, d_bias, bias_dtype, d_y, y_dtype, ldy, &a, &run));
   if (!run) return TMH_OK;
-  // The call keeps its scratch memory within the scratch area: GM_SPLIT's rows of A when they fit
-  // (else the general kernel runs), then the partial sums of the best plan that fits in the rest
-  // (where tmh_matmul_nbits's plan would need more: fewer splits of K, or none).
+  // The call keeps its scratch memory within the scratch area: the split rows of A when they fit (else
+  // the route without the prefill GEMM: k_gemv_rows, or k_matmul_general), then the partial sums of the
+  // best plan that fits in the rest (where tmh_matmul_nbits's plan would need more: fewer splits of K,
+  // or none).
   if (splits_a(gemm_mode(w, a)) && split_a_bytes(w, a.M) > kNoallocScratchBytes) a.no_split_a = true;
   const size_t rows_a = splits_a(gemm_mode(w, a)) ? split_a_bytes(w, a.M) : 0;
   a.split_cap = kNoallocScratchBytes - rows_a;
