@@ -81,7 +81,8 @@ def test_launch_shapes(ctx, m, n, chunks, a_dtype, w_dtype):
 # lane's group.
 @pytest.mark.parametrize("a_dtype,w_dtype", TYPES)
 @pytest.mark.parametrize("bits,block", [(2, 16), (2, 64), (4, 16), (8, 32)])
-@pytest.mark.parametrize("m,n,chunks", [(16, 4160, 9), (16, 33000, 2), (20, 5000, 3), (48, 2704, 2), (30, 16500, 2), (64, 16200, 3)])
+@pytest.mark.parametrize("m,n,chunks", [(16, 4160, 9), (16, 33000, 2), (20, 5000, 3), (48, 2704, 2), (30, 16500, 2), (64, 16200, 3),
+                                        (24, 5000, 5), (24, 5000, 9), (40, 5000, 9)])
 def test_launch_shapes_of_other_weights(ctx, m, n, chunks, bits, block, a_dtype, w_dtype):
     k = chunks * chunk(bits) - 24
     print(f"rows m={m} n={n} k={k} b{bits} bs{block} {a_dtype}", flush=True)

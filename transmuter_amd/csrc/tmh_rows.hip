@@ -42,9 +42,15 @@ void launch_op(const RowsArgs& d, int64_t M, const RowsPlan& p, hipStream_t s) {
   if constexpr (OP != ROW_GEN) {
     TMH_ROWS(1, 2, 8);
     TMH_ROWS(2, 2, 8);
+    if constexpr (BITS == 2 && SPLIT) {
+      TMH_ROWS(1, 1, 4);
+      TMH_ROWS(2, 2, 2);
+    } else {
+      TMH_ROWS(1, 2, 4);
+    }
+    if constexpr (BITS != 2 && SPLIT) TMH_ROWS(2, 2, 4);
     if constexpr (BITS != 2 && !SPLIT) {
       TMH_ROWS(1, 1, 16);
-      TMH_ROWS(1, 2, 4);
       if constexpr (OP != ROW_INT) {
         TMH_ROWS(1, 2, 16);
         TMH_ROWS(2, 2, 4);
@@ -71,13 +77,34 @@ void launch_op(const RowsArgs& d, int64_t M, const RowsPlan& p, hipStream_t s) {
 //  - beyond, the workgroups come in rounds: four wavefronts with more chunks each keep their loads
 //    going (bf16 1024->151936, M = 12: 1,2,4 27.4, 1,2,8 34.1; f32 2048->22016, M = 12: 1,2,4 20.4,
 //    1,2,8 25.2; f16 2048->22016, M = 24: 2,2,4 14.8, 1,2,8 16.5, 2,4,8 16.7).
-// 2-bit weights and parameters that change within a lane's group hold more registers per tile.
-RowsPlan plan_rows(int op, bool wide_regs, int64_t M, int64_t ntiles, int64_t nch, int cus) {
+// 8 bits lie the same way (of 35 sizes none has a shape over 6% faster). 2-bit weights and parameters that
+// change within a lane's group hold more registers per tile: two tiles at most, and with few chunks of K
+// fewer wavefronts, as idle ones keep other workgroups off the CU:
+//  - 2 bits (f16): M = 64 512->16000 1,2,4 8.4, 1,2,8 15.7, 2,2,8 10.4; 1024->6144 5.8, 8.5, 9.7; 2048->8192
+//    12.1, 15.1, 27.4; one set of rows and eight chunks 1,2,8 5.0, 1,2,4 5.3. With 17 or 18 rows the second
+//    set is nearly free (bf16 M = 17 2048->8192 2,2,8 7.6, 1,2,4 8.4);
+//  - 2 bits in blocks of 16 or 32: M = 64 512->16000 2,2,2 10.0, 1,1,4 12.9, 1,2,8 20.8; 1024->6144 1,1,4 9.1,
+//    2,2,2 10.0, 1,2,8 10.7; 2048->8192 1,2,8 17.8, 1,1,4 21.5, 2,2,2 31.9; up to four workgroups a CU M = 32
+//    768->5000 2,2,8 5.5, 2,2,2 6.1;
+//  - 4 bits in blocks of 16: M = 64 512->16000 2,2,4 8.4, 2,2,8 12.4, 1,2,4 10.2; 2048->8192 11.9, 13.7, 14.0;
+//    M = 20 512->16000 4.8, 6.5, 6.4; 2048->8192 7.0, 6.8, 7.9; M = 8 512->16000 1,2,4 4.4, 1,2,8 5.3, six
+//    chunks 4.2, 4.0.
+RowsPlan plan_rows(int op, int bits, bool split, int64_t M, int64_t ntiles, int64_t nch, int cus) {
   const int64_t r = (M + 15) / 16, work = ntiles * r;
   const int nw = nch > 8 ? 16 : 8;
+  const bool wide_regs = bits == 2 || split;
   if (op == ROW_GEN) return {1, 1, 8};
   if (work <= cus) return {1, 1, wide_regs ? 8 : nw};
-  if (wide_regs) return r == 1 || work <= 2 * cus ? RowsPlan{1, 2, 8} : RowsPlan{2, 2, 8};
+  if (wide_regs) {
+    const bool few = nch < (bits == 2 ? 8 : 5), barely = r == 2 && M <= 18;
+    if (r == 1 || work <= 2 * cus) return {1, 2, few && !(bits == 2 && split) ? 4 : 8};
+    if (bits == 2 && split) {
+      if (barely || (few && work <= 4 * cus)) return {2, 2, 8};
+      return nch <= 3 ? RowsPlan{2, 2, 2} : few ? RowsPlan{1, 1, 4} : RowsPlan{1, 2, 8};
+    }
+    if (bits == 2) return barely ? RowsPlan{2, 2, 8} : RowsPlan{1, 2, 4};
+    return {2, 2, r == 2 && !few ? 8 : 4};
+  }
   if (op == ROW_INT) {
     if (work <= 2 * cus) return {1, 2, 8};
     if (r > 1 && work <= 4 * cus) return {2, 2, 8};
@@ -128,7 +155,7 @@ void launch_rows(const tmh_weight* w, const void* a, int a_dtype, int64_t M, int
                    static_cast<uint32_t>(y_dtype) | (static_cast<uint32_t>(dot_dtype) << 8) |
                        (static_cast<uint32_t>(bias ? bias_dtype : 0) << 16) | (static_cast<uint32_t>(a_dtype) << 24),
                    static_cast<uint32_t>(w->zp_kind) | (static_cast<uint32_t>(w->wdtype) << 8), bias};
-  const RowsPlan p = plan_rows(op, w->bits == 2 || split, M, w->ntiles, w->nchunks, num_cus > 0 ? num_cus : 256);
+  const RowsPlan p = plan_rows(op, w->bits, split, M, w->ntiles, w->nchunks, num_cus > 0 ? num_cus : 256);
 #define TMH_ROWS_BITS(B)                                                          \
   switch (op) {                                                                   \
     case ROW_F16:                                                                 \
