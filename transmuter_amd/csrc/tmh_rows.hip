@@ -183,7 +183,7 @@ void launch_rows(const tmh_weight* w, const void* a, int a_dtype, int64_t M, int
 
 // As many rows a launch as its shape and 32-bit offsets over A take: a launch for every 64 rows would
 // leave the chip idle where N is small (bf16 in blocks of 16, us: 16384 x 64 -> 64 k_matmul_general 218,
-// a launch for every 64 rows 516, this 14.5; 1024 x 2048 -> 2048 2390, 93, 53).
+// a launch for every 64 rows 516, this 14.1; 1024 x 2048 -> 2048 2390, 93, 37).
 void launch_gemv_rows(const tmh_weight* w, const void* a, int a_dtype, int64_t M, int64_t lda, const void* bias,
                       int bias_dtype, void* y, int y_dtype, int dot_dtype, int64_t ldy, hipStream_t s, int num_cus) {
   const int64_t a_size = dtype_size(a_dtype), fit = ((int64_t(1) << 31) - 1) / (lda * a_size) / 64 * 64;
